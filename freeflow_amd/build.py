@@ -20,7 +20,9 @@ LIB = os.path.join(PKG, "lib")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-HIP_SOURCES = ["capi.hip", "kernels2d.hip", "kernels3d.hip", "links.hip", "batch.hip"]
+HIP_SOURCES = ["capi.hip", "kernels2d.hip", "links.hip"]
+# compiled once per storage format (FF_TU_STORAGE): they instantiate every tile shape
+STORAGE_SOURCES = ["kernels3d.hip", "batch.hip"]
 
 # -ffp-contract=off: the 2D path reproduces the reference's FP32 rounding
 # (including its FP16 tile staging) and the link predicates take discrete
@@ -46,10 +48,12 @@ def build_hip_lib(jobs=8):
     os.makedirs(LIB, exist_ok=True)
     objs = []
     cmds = []
-    for src in HIP_SOURCES:
-        o = os.path.join(OBJ, src.replace(".hip", ".o"))
+    units = [(src, k) for src in STORAGE_SOURCES for k in range(4)] + [(src, None) for src in HIP_SOURCES]
+    for src, k in units:
+        o = os.path.join(OBJ, src.replace(".hip", ".o" if k is None else f"_s{k}.o"))
         objs.append(o)
-        cmds.append([HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, src), "-o", o])
+        define = [] if k is None else [f"-DFF_TU_STORAGE={k}"]
+        cmds.append([HIPCC, *HIP_FLAGS, *define, "-c", os.path.join(CSRC, src), "-o", o])
     with cf.ThreadPoolExecutor(max_workers=min(jobs, len(cmds))) as ex:
         for out in ex.map(_run, cmds):
             if out:

@@ -108,16 +108,6 @@ constexpr int kDirectSteps = 4;
 constexpr int kGraphSteps = 8;
 
 // ---------------------------------------------------------------- kernels
-// A pointer read from the domain table lies in device global memory, but
-// being read from memory (not passed as a kernel argument) the compiler
-// cannot tell, and addresses it generically (flat instructions, which also
-// count against the LDS wait counter).  Passed through an integer into the
-// global address space, every access derived from it is a global one.
-template <typename T>
-__device__ __forceinline__ T* dev_global(T* p) {
-  return (T*)(__attribute__((address_space(1))) T*)reinterpret_cast<unsigned long long>(p);
-}
-
 // Stream launch: [boundary-cell blocks of every domain][wave blocks][tiles].
 template <typename S, bool STAGE, bool PERIODIC, int TX, int TY, int CPT, bool FAST>
 __global__ void __launch_bounds__(256) kb_step2d(const DomDev* __restrict__ doms, const int2* __restrict__ map,
@@ -195,28 +185,7 @@ __global__ void __launch_bounds__(FB) kb_finish(const DomDev* __restrict__ doms,
   if (threadIdx.x == 0) *D->step = *D->step + 1u;
 }
 
-// Pending detections: tag bumps of members whose earlier detection went
-// stale, then the detection blocks of every pending member (one launch for
-// the whole batch instead of one per domain).
-__global__ void kb_tag_bump(const DomDev* __restrict__ doms, const int2* __restrict__ list, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) {
-    StepState* st = doms[list[i].x].la.st;
-    st->tag = st->tag + 1u;
-  }
-}
-
-template <int DIM>
-__global__ void __launch_bounds__(kSumBlock) kb_detect(const DomDev* __restrict__ doms, const int2* __restrict__ map) {
-  const int2 m = map[blockIdx.x];
-  const LinkArgs& la = doms[m.x].la;
-  detect_block<DIM>(la, (long long)m.y, step_tag(la), la.v[step_gen(la) & 1u]);
-}
-
 // ---------------------------------------------------------------- launch helpers
-// Block size of the stream launch for a tile index.
-static int stream_threads(int dim, int tile) { return dim == 2 ? 256 : kTiles3[tile].nt; }
-
 template <typename S, bool STAGE, bool PERIODIC, int TX, int TY, int CPT, bool FAST>
 static void step2d_batch_shape(Batch& b, const int2* map, int nblocks, int n_bc, int n_wave) {
   launch_timed(kb_step2d<S, STAGE, PERIODIC, TX, TY, CPT, FAST>, dim3(nblocks), dim3(256), b.stream, b.tev0, b.tev1,
@@ -250,7 +219,7 @@ static void step3d_batch_variant(Batch& b, int tile, const int2* map, int nblock
 
 // The stream launch over `map` (n_bc boundary-cell blocks, n_wave wave blocks, then tiles).
 template <typename S>
-static void launch_stream_batch(Batch& b, int tile, const int2* map, int nblocks, int n_bc, int n_wave) {
+void launch_stream_batch(Batch& b, int tile, const int2* map, int nblocks, int n_bc, int n_wave) {
   if (nblocks <= 0) return;
   const bool stage = b.options & FF_OPT_STAGE_FP16, per = b.options & FF_OPT_PERIODIC;
   const bool fast = b.options & FF_OPT_FAST_MATH;
@@ -278,7 +247,7 @@ static void launch_tail(Batch& b, const int2* map_sums, const int2* map_fin) {
 }
 
 template <typename S>
-static void launch_step_typed(Batch& b, int tile) {
+void launch_step_typed(Batch& b, int tile) {
   const int n_stream = b.n_bc + b.n_wave + b.n_bulk;
   const int2* map_stream = b.d_map;
   const int2* map_sums = map_stream + n_stream;
@@ -287,6 +256,43 @@ static void launch_step_typed(Batch& b, int tile) {
   if (b.dim == 2) launch_tail<2, S>(b, map_sums, map_fin);
   else launch_tail<3, S>(b, map_sums, map_fin);
 }
+
+template void launch_stream_batch<tu_storage>(Batch&, int, const int2*, int, int, int);
+template void launch_step_typed<tu_storage>(Batch&, int);
+
+}  // namespace ff
+
+#if FF_TU_STORAGE == 0
+namespace ff {
+
+#define FF_ELSEWHERE(S)                                                                     \
+  extern template void launch_stream_batch<S>(Batch&, int, const int2*, int, int, int); \
+  extern template void launch_step_typed<S>(Batch&, int);
+FF_ELSEWHERE(__half)
+FF_ELSEWHERE(__hip_bfloat16)
+FF_ELSEWHERE(h16u)
+#undef FF_ELSEWHERE
+
+// Pending detections: tag bumps of members whose earlier detection went
+// stale, then the detection blocks of every pending member (one launch for
+// the whole batch instead of one per domain).
+__global__ void kb_tag_bump(const DomDev* __restrict__ doms, const int2* __restrict__ list, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) {
+    StepState* st = doms[list[i].x].la.st;
+    st->tag = st->tag + 1u;
+  }
+}
+
+template <int DIM>
+__global__ void __launch_bounds__(kSumBlock) kb_detect(const DomDev* __restrict__ doms, const int2* __restrict__ map) {
+  const int2 m = map[blockIdx.x];
+  const LinkArgs& la = doms[m.x].la;
+  detect_block<DIM, true>(la, (long long)m.y, step_tag(la), la.v[step_gen(la) & 1u]);
+}
+
+// Block size of the stream launch for a tile index.
+static int stream_threads(int dim, int tile) { return dim == 2 ? 256 : kTiles3[tile].nt; }
 
 static void launch_step(Batch& b, int tile) {
   if (b.storage == FF_STORAGE_F32) launch_step_typed<float>(b, tile);
@@ -370,13 +376,13 @@ static int build_tables(Batch& b, int tile) {
         for (int t = 0; t < nw; t++) wave.push_back(make_int2(i, t));
       }
       r.nvb = (d.nv + 255) / 256;
-      r.ndet = detect_blocks(d, kSumBlock, true);
+      r.ndet = detect_blocks(d, true);
       r.fa.copy_blocks = copyback_blocks(d, kSumBlock, 4);  // fewer blocks: many domains share the launch
     } else {
       r.la.ne = 0;
       r.fa.copy_blocks = 0;
     }
-    const int nes = (bnd ? elem_blocks(d.ne) : 0) + r.fa.outlet_blocks + r.fa.copy_blocks + r.ndet;
+    const int nes = (bnd ? elem_blocks(b.dim, d.ne) : 0) + r.fa.outlet_blocks + r.fa.copy_blocks + r.ndet;
     for (int t = 0; t < nes; t++) es.push_back(make_int2(i, t));
     for (int t = 0; t <= r.nvb; t++) fin.push_back(make_int2(i, t));
   }
@@ -591,7 +597,7 @@ static int detect_pending(Batch& b) {
       b.bumps.push_back(make_int2((int)i, 0));
       d.tag_host++;  // mirror of the device bump
     }
-    const int nd = detect_blocks(d, kSumBlock, true);
+    const int nd = detect_blocks(d, true);
     for (int t = 0; t < nd; t++) b.dets.push_back(make_int2((int)i, t));
     d.stale = false;
     d.predetected = true;
@@ -840,3 +846,5 @@ int ff_batch_time_bulk(ff_batch* b, int iters, double* avg_ms) {
 }
 
 }  // extern "C"
+
+#endif  // FF_TU_STORAGE == 0

@@ -235,6 +235,7 @@ int launch_wave_now(Domain& d);
 // and 8 FP32 values derived from them for the fast-math kinematics.
 constexpr int kWaveParStride = 8;  // doubles per body
 void wave_device_params(const double* p4, double dt, int n_bodies, double* out);
+int detect_blocks(const Domain& d, bool batched);  // detection blocks of 256 threads
 int bc_span(const Domain& d);  // boundary-cell scan span of a domain stepped on its own
 int launch_step_vertex_forces(Domain& d, float* out_dev);
 int launch_convert_in(Domain& d, const float* aos_dev, void* buf);

@@ -35,14 +35,31 @@ __device__ __forceinline__ unsigned mix32(unsigned h) {
 __device__ __forceinline__ unsigned step_gen(const LinkArgs& la) { return la.dev_state ? la.st->gen : la.gen; }
 __device__ __forceinline__ unsigned step_tag(const LinkArgs& la) { return la.dev_state ? la.st->tag : la.tag; }
 
+// A pointer read from a record in device memory (the batch's domain table) is
+// not known to be global to the compiler, which then addresses it generically
+// (flat instructions, which also count against the LDS wait counter).  Passed
+// through an integer into the global address space, every access derived from
+// it is a global one; a pointer that is a kernel argument is unchanged.
+template <typename T>
+__device__ __forceinline__ T* dev_global(T* p) {
+  return (T*)(__attribute__((address_space(1))) T*)reinterpret_cast<unsigned long long>(p);
+}
+
+// Two adjacent 4-byte values in one load.  A caller's own boundary arrays
+// (ff_step_proxy) are only 4-byte aligned, and these types say so.
+typedef float f32x2 __attribute__((ext_vector_type(2), aligned(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ f32x2 load2(const float* p) { return *reinterpret_cast<const f32x2*>(p); }
+__device__ __forceinline__ u32x2 load2(const uint32_t* p) { return *reinterpret_cast<const u32x2*>(p); }
+
 // Two link tables alternate by tag parity: the next step's links are detected
 // into one while the current step's are read from the other.
 __device__ __forceinline__ unsigned long long* table_cells(const LinkArgs& la, unsigned tag) {
-  return la.cells + (size_t)(tag & 1u) * la.cap;
+  return dev_global(la.cells) + (size_t)(tag & 1u) * la.cap;
 }
 template <int DIM>
 __device__ __forceinline__ unsigned long long* table_keys(const LinkArgs& la, unsigned tag) {
-  return la.keys + (size_t)(tag & 1u) * la.cap * (DIM == 2 ? 8 : 26);
+  return dev_global(la.keys) + (size_t)(tag & 1u) * la.cap * (DIM == 2 ? 8 : 26);
 }
 
 // Slot of `cell` under generation `gen`, entering it if absent.  The cells of
@@ -65,16 +82,25 @@ __device__ __forceinline__ int lt_claim(unsigned long long* cells, int cap, unsi
   return -1;
 }
 
-__device__ __forceinline__ int lt_find(const unsigned long long* cells, int cap, unsigned gen, int cell) {
+__device__ __forceinline__ unsigned lt_home(int cap, int cell) { return mix32((unsigned)cell) & (unsigned)(cap - 1); }
+
+// Slot of `cell` or -1; `h` is its home slot and `cur` that slot's word (the
+// caller loads it, so the loads of several cells are in flight together).
+__device__ __forceinline__ int lt_resolve(const unsigned long long* cells, int cap, unsigned gen, int cell, unsigned h,
+                                          unsigned long long cur) {
   const unsigned long long want = ((unsigned long long)gen << 32) | (unsigned)cell;
-  unsigned h = mix32((unsigned)cell) & (unsigned)(cap - 1);
   for (int probe = 0; probe < cap; probe++) {
-    const unsigned long long cur = cells[h];
     if (cur == want) return (int)h;
     if ((unsigned)(cur >> 32) != gen) return -1;
     h = (h + 1) & (unsigned)(cap - 1);
+    cur = cells[h];
   }
   return -1;
+}
+
+__device__ __forceinline__ int lt_find(const unsigned long long* cells, int cap, unsigned gen, int cell) {
+  const unsigned h = lt_home(cap, cell);
+  return lt_resolve(cells, cap, gen, cell, h, cells[h]);
 }
 
 __device__ __forceinline__ void lt_offer_key(unsigned long long* keys, size_t idx, unsigned gen, uint32_t key) {
@@ -107,6 +133,17 @@ __device__ __forceinline__ float seg_link(float x1, float y1, float x2, float y2
     return (float)(1.0 - (double)t1);
   }
   return -1.0f;
+}
+
+// Superset, without a division, of "t1 = b1 / a1 lies in (0, 1)" (the line
+// test of seg_link): the quotient is positive only if b1 is nonzero with a1's
+// sign, and rounds below 1 only if |b1| < |a1| (rounding is monotone and 1 is
+// representable); NaN operands compare false here and fail there.
+__device__ __forceinline__ bool seg_link_may_hit(float x1, float y1, float x2, float y2, float x3, float y3, float x4,
+                                                 float y4) {
+  const float a1 = (x1 - x2) * (y3 - y4) - (y1 - y2) * (x3 - x4);
+  const float b1 = (x4 - x2) * (y3 - y4) - (y4 - y2) * (x3 - x4);
+  return fabsf(b1) < fabsf(a1) && b1 != 0.0f && (b1 > 0.0f) == (a1 > 0.0f);
 }
 
 struct Hit {
@@ -240,6 +277,18 @@ __device__ __forceinline__ void elem_window(const float* v, const uint32_t* e, i
   }
 }
 
+// elem_window<2> of a segment given by its end points.
+__device__ __forceinline__ void seg_window(f32x2 a, f32x2 b, float dx, const int* n, int* lo, int* hi) {
+  const float c[2][2] = {{a.x, b.x}, {a.y, b.y}};
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const float mn = fminf(fminf(FLT_MAX, c[k][0]), c[k][1]);
+    const float mx = fmaxf(fmaxf(FLT_MIN, c[k][0]), c[k][1]);
+    lo[k] = max((int)(mn / dx) - 1, 0);
+    hi[k] = min((int)(mx / dx) + 1, n[k] - 1);
+  }
+}
+
 }  // namespace ff
 
 #include "ff_internal.h"
@@ -258,111 +307,119 @@ constexpr unsigned long long d3_pack(int axis) {
 }
 __device__ __forceinline__ int d3_c(unsigned long long packed, int i) { return (int)((packed >> (2 * i)) & 3ull) - 1; }
 
-// Lanes that detect one element's links in a batch (many domains: whole
-// elements per lane group need fewer blocks for the same work).
-template <int DIM>
-constexpr int kDetectLanes = DIM == 2 ? 32 : 256;
+// Lanes that handle one element in the 2D detection and element sums: a DPP
+// row.  A segment's candidate window holds 9-20 cells (segments of 0.4-1.5
+// cells), so 16 lanes take it in one or two passes and a wave works on four
+// elements; with a wave or half a wave per element most lanes had no cell.
+constexpr int kRow = 16;
 
-// 2D link detection: a group of LPE lanes per element walks the element's
-// candidate window once for every lattice direction, one (window cell,
-// direction) task per lane (the loops of mrSolver2DComputeOccupancyFlagKernel_v3,
-// FsiCoupling2D.cu:44-74), and offers depthIndexCompact keys for every hit of
-// an updated cell.  `block` indexes groups of blockDim / LPE elements; the
-// links are entered under `tag` for the vertex positions `v`.
-template <int LPE>
-__device__ __forceinline__ void build_links_block2(const LinkArgs& la, long long block, unsigned tag, const float* v) {
-  const unsigned gen = tag;
+// Lattice vectors of D2Q9 packed two bits per direction (c + 1).
+constexpr unsigned d2_pack(int axis) {
+  unsigned p = 0;
+  for (int i = 0; i < 9; i++) p |= (unsigned)((axis == 0 ? D2::cx(i) : D2::cy(i)) + 1) << (2 * i);
+  return p;
+}
+
+// 2D link detection (the loops of mrSolver2DComputeOccupancyFlagKernel_v3,
+// FsiCoupling2D.cu:44-74): kRow lanes per element, one window cell per lane
+// and pass.  A lane tests its cell's eight links against the segment's line
+// without a division (seg_link_may_hit), finishes the survivors, enters the
+// cell once if any link hit, and offers the hits' depthIndexCompact keys.
+// Bound by the chain of dependent loads (element -> vertices -> flags -> table)
+// and by instruction issue: with one (cell, direction) task per lane every
+// task divided, and every hit walked the table by itself.
+// `block` indexes groups of blockDim / kRow elements; the links are entered
+// under `tag` for the vertex positions `v`.
+__device__ __forceinline__ void build_links_rows2(const LinkArgs& la, long long block, unsigned tag, const float* v) {
   constexpr int K = 8;
-  const long long e = block * (long long)(blockDim.x / LPE) + threadIdx.x / LPE;
+  const long long e = block * (long long)(blockDim.x / kRow) + threadIdx.x / kRow;
   if (e >= (long long)la.ne) return;
-  const int elem = (int)e, lane = (int)(threadIdx.x % LPE);
-  const int n[3] = {la.nx, la.ny, la.nz};
-  int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-  elem_window<2>(v, la.e, elem, la.cl, n, lo, hi);
+  const int lane = (int)(threadIdx.x % kRow);
+  const u32x2 ends = load2(dev_global(la.e) + 2 * e);
+  const f32x2 p3 = load2(dev_global(v) + 2 * (size_t)ends.x), p4 = load2(dev_global(v) + 2 * (size_t)ends.y);
+  const int n[2] = {la.nx, la.ny};
+  int lo[2], hi[2];
+  seg_window(p3, p4, la.cl, n, lo, hi);
   const int wx = hi[0] - lo[0] + 1, wy = hi[1] - lo[1] + 1;
   if (wx <= 0 || wy <= 0) return;
-  const int ntask = wx * wy * K;
-  const uint32_t sa = la.e[2 * elem], sb = la.e[2 * elem + 1];
-  const float p3x = v[2 * sa], p3y = v[2 * sa + 1], p4x = v[2 * sb], p4y = v[2 * sb + 1];
-  unsigned long long* cells = table_cells(la, gen);
-  unsigned long long* keys = table_keys<2>(la, gen);
-  for (int t = lane; t < ntask; t += LPE) {
-    const int k = t / K;
-    const int l = t - k * K + 1;
-    const int i = lo[0] + k % wx, j = lo[1] + k / wx;
+  const int ncell = wx * wy;
+  const uint8_t* flags = dev_global(la.flags);
+  unsigned long long* cells = table_cells(la, tag);
+  unsigned long long* keys = table_keys<2>(la, tag);
+  for (int k = lane; k < ncell; k += kRow) {
+    const int j0 = k / wx;
+    const int i = lo[0] + k - j0 * wx, j = lo[1] + j0;
+    const int cell = j * la.nx + i;
+    if (!is_updated(flags[cell])) continue;
+    const float fi = (float)i, fj = (float)j, x1 = fi * la.cl, y1 = fj * la.cl;
+    unsigned may = 0;
+#pragma unroll
+    for (int l = 1; l <= K; l++)
+      if (seg_link_may_hit(x1, y1, (fi - (float)D2::cx(l)) * la.cl, (fj - (float)D2::cy(l)) * la.cl, p3.x, p3.y, p4.x,
+                           p4.y))
+        may |= 1u << l;
+    auto test = [&](int l, Hit& h) {
+      const float cx = (float)((int)((d2_pack(0) >> (2 * l)) & 3u) - 1);
+      const float cy = (float)((int)((d2_pack(1) >> (2 * l)) & 3u) - 1);
+      return hit_seg2(p3.x, p3.y, p4.x, p4.y, x1, y1, (fi - cx) * la.cl, (fj - cy) * la.cl, h);
+    };
+    unsigned hits = 0;
+    for (unsigned m = may; m; m &= m - 1) {
+      const int l = __ffs((int)m) - 1;
+      Hit h;
+      if (test(l, h)) hits |= 1u << l;
+    }
+    if (!hits) continue;
+    const int slot = lt_claim(cells, la.cap, tag, cell, &la.st->overflow);
+    if (slot < 0) continue;
+    for (unsigned m = hits; m; m &= m - 1) {
+      const int l = __ffs((int)m) - 1;
+      Hit h;
+      test(l, h);
+      lt_offer_key(keys, (size_t)slot * K + (l - 1), tag, depth_key(h.depth, (int)e));
+    }
+  }
+}
+
+// 2D link detection of a domain stepped on its own: kRow lanes per (element,
+// direction), one window cell per lane.  Eight times the waves of
+// build_links_rows2 for the same predicates, hits and keys, and the shorter
+// chain (one test and one table walk per lane), which is what a launch of few
+// blocks waits for: 5.6 us against 7.4 us for the 600 segments of a 1200x400
+// swimmer; with 64 domains (26.9 against 16.9 us) the launch is bound by issue.
+// `block` indexes groups of blockDim / kRow pairs.
+__device__ __forceinline__ void build_links_pairs2(const LinkArgs& la, long long block, unsigned tag, const float* v) {
+  constexpr int K = 8;
+  const int lane = (int)(threadIdx.x % kRow);
+  const long long pair = block * (long long)(blockDim.x / kRow) + threadIdx.x / kRow;
+  if (pair >= (long long)la.ne * K) return;
+  const int elem = (int)(pair / K), l = (int)(pair % K) + 1;
+  const u32x2 ends = load2(la.e + 2 * (size_t)elem);
+  const f32x2 p3 = load2(v + 2 * (size_t)ends.x), p4 = load2(v + 2 * (size_t)ends.y);
+  const int n[2] = {la.nx, la.ny};
+  int lo[2], hi[2];
+  seg_window(p3, p4, la.cl, n, lo, hi);
+  const int wx = hi[0] - lo[0] + 1, wy = hi[1] - lo[1] + 1;
+  if (wx <= 0 || wy <= 0) return;
+  const int ncell = wx * wy;
+  const float cx = (float)D2::cx(l), cy = (float)D2::cy(l);
+  unsigned long long* cells = table_cells(la, tag);
+  unsigned long long* keys = table_keys<2>(la, tag);
+  for (int k = lane; k < ncell; k += kRow) {
+    const int j0 = k / wx;
+    const int i = lo[0] + k - j0 * wx, j = lo[1] + j0;
     const int cell = j * la.nx + i;
     Hit h;
-    bool hit = false;
-    if (is_updated(la.flags[cell]))
-      hit = hit_seg2(p3x, p3y, p4x, p4y, (float)i * la.cl, (float)j * la.cl, ((float)i - (float)D2::cx(l)) * la.cl,
-                     ((float)j - (float)D2::cy(l)) * la.cl, h);
-    const int slot = hit ? lt_claim(cells, la.cap, gen, cell, &la.st->overflow) : -1;
-    if (slot >= 0) lt_offer_key(keys, (size_t)slot * K + (l - 1), gen, depth_key(h.depth, elem));
+    const bool hit = is_updated(la.flags[cell]) &&
+                     hit_seg2(p3.x, p3.y, p4.x, p4.y, (float)i * la.cl, (float)j * la.cl, ((float)i - cx) * la.cl,
+                              ((float)j - cy) * la.cl, h);
+    const int slot = hit ? lt_claim(cells, la.cap, tag, cell, &la.st->overflow) : -1;
+    if (slot >= 0) lt_offer_key(keys, (size_t)slot * K + (l - 1), tag, depth_key(h.depth, elem));
   }
 }
 
-// Link detection with one 16-lane group per (element, direction) pair, each
-// lane one window cell: the shortest latency for a domain stepped on its own
-// (the same predicates, hits and keys as build_links_block2 and
-// build_links_block3).  `block` indexes
-// groups of blockDim / 16 pairs.
-template <int DIM>
-__device__ __forceinline__ void build_links_pairs(const LinkArgs& la, long long block, unsigned tag, const float* v) {
-  const unsigned gen = tag;
-  constexpr int K = DIM == 2 ? 8 : 26;
-  const int lane = threadIdx.x & 15;
-  const long long pair = block * (blockDim.x >> 4) + (threadIdx.x >> 4);
-  if (pair >= (long long)la.ne * K) return;
-  const int elem = (int)(pair / K);
-  const int l = (int)(pair % K) + 1;
-  const int n[3] = {la.nx, la.ny, la.nz};
-  int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-  elem_window<DIM>(v, la.e, elem, la.cl, n, lo, hi);
-  const int wx = hi[0] - lo[0] + 1, wy = hi[1] - lo[1] + 1, wz = DIM == 3 ? hi[2] - lo[2] + 1 : 1;
-  if (wx <= 0 || wy <= 0 || wz <= 0) return;
-  const int ncell = wx * wy * wz;
-  const int cx = DIM == 2 ? D2::cx(l) : d3_c(d3_pack(0), l);
-  const int cy = DIM == 2 ? D2::cy(l) : d3_c(d3_pack(1), l);
-  const int cz = DIM == 2 ? 0 : d3_c(d3_pack(2), l);
-  unsigned long long* cells = table_cells(la, gen);
-  unsigned long long* keys = table_keys<DIM>(la, gen);
-  Tri3 T;
-  float p3x = 0.f, p3y = 0.f, p4x = 0.f, p4y = 0.f;
-  if constexpr (DIM == 3) {
-    T = tri3(v, la.e, elem);
-  } else {
-    const uint32_t sa = la.e[2 * elem], sb = la.e[2 * elem + 1];
-    p3x = v[2 * sa];
-    p3y = v[2 * sa + 1];
-    p4x = v[2 * sb];
-    p4y = v[2 * sb + 1];
-  }
-  for (int k = lane; k < ncell; k += 16) {
-    const int i = lo[0] + k % wx;
-    const int j = lo[1] + (k / wx) % wy;
-    const int z = DIM == 3 ? lo[2] + k / (wx * wy) : 0;
-    const int cell = (z * la.ny + j) * la.nx + i;
-    Hit h;
-    bool hit = false;
-    if (is_updated(la.flags[cell])) {
-      if constexpr (DIM == 2) {
-        hit = hit_seg2(p3x, p3y, p4x, p4y, (float)i * la.cl, (float)j * la.cl, ((float)i - (float)cx) * la.cl,
-                       ((float)j - (float)cy) * la.cl, h);
-      } else {
-        const float p1[3] = {(float)i * la.cl, (float)j * la.cl, (float)z * la.cl};
-        const float p2[3] = {((float)i - (float)cx) * la.cl, ((float)j - (float)cy) * la.cl,
-                             ((float)z - (float)cz) * la.cl};
-        hit = hit_tri3(T, p1, p2, h);
-      }
-    }
-    const int slot = hit ? lt_claim(cells, la.cap, gen, cell, &la.st->overflow) : -1;
-    if (slot >= 0) lt_offer_key(keys, (size_t)slot * K + (l - 1), gen, depth_key(h.depth, elem));
-  }
-}
-
-// Survivor capacity of build_links_block3's LDS lists (an int and a byte
-// each).
-constexpr int kDet3Cap = 2048;
+// Capacity of build_links_block3's LDS lists.
+constexpr int kDet3Cap = 4096;
 
 // Superset test, without a division, of "num / den rounds into [0, 1] or is
 // NaN" (the plane-parameter test of line_triangle_intersect): num = 0 gives
@@ -378,122 +435,148 @@ __device__ __forceinline__ bool tri3_t_may_pass(float num, float den) {
 }
 
 // 3D link detection with one 256-thread block per element, cell-major: each
-// thread takes one cell of the element's window per pass (window coordinates
-// formed once per cell), forms num = n . (v0 - p1), and only cells within
-// 2 cl of the triangle's plane go on (no link of length <= sqrt(3) cl from a
-// farther cell reaches it; the margin is far above the rounding of the link
-// ends for grids up to millions of cells per axis).  For each of the 26
-// directions (unrolled, lattice vectors as constants) links whose plane
-// parameter t = num / (n . dd) may lie in [0, 1] (tri3_t_may_pass, no
-// division) are gathered in LDS; once the lists may fill, and at the end, the
-// block finishes them (t itself, parallel test, barycentrics, table entry).
-// Same predicates, hits and keys as build_links_pairs.
+// thread takes two cells of the element's window per pass, forms
+// num = n . (v0 - p1), and only cells within 2 cl of the triangle's plane go
+// on (no link of length <= sqrt(3) cl from a farther cell reaches it; the
+// margin is far above the rounding of the link ends for grids up to millions
+// of cells per axis).  Their 26 links (unrolled, lattice vectors as constants)
+// whose plane parameter t = num / (n . dd) may lie in [0, 1] (tri3_t_may_pass,
+// no division) form a bit mask; a block-wide prefix sum of the masks' counts
+// lists the survivors in LDS, all threads finish them (t itself, parallel
+// test, barycentrics), and the hits, listed again, are entered in the table
+// together.  Bound by the chain of loads, barriers and table round trips of
+// one block: one list position per direction from an LDS counter, with a
+// barrier every fourth, took 21 us for the 320 triangles of a sphere.
 __device__ __forceinline__ void build_links_block3(const LinkArgs& la, long long block, unsigned tag, const float* v) {
-  constexpr int K = 26;
-  constexpr int NT = 256;
-  __shared__ int s_n;
-  __shared__ int s_cell[kDet3Cap];
-  __shared__ unsigned char s_dir[kDet3Cap];
+  constexpr int K = 26, NT = 256, NW = NT / 64, U = 2;
+  __shared__ int s_wave[NW], s_nhit;
+  __shared__ unsigned short s_may[kDet3Cap], s_hit[kDet3Cap];
   if (block >= (long long)la.ne) return;  // block-uniform
-  const unsigned gen = tag;
   const int elem = (int)block;
   const int n[3] = {la.nx, la.ny, la.nz};
-  int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-  elem_window<3>(v, la.e, elem, la.cl, n, lo, hi);
+  const uint32_t* e = dev_global(la.e);
+  v = dev_global(v);
+  int lo[3], hi[3];
+  elem_window<3>(v, e, elem, la.cl, n, lo, hi);
   const int wx = hi[0] - lo[0] + 1, wy = hi[1] - lo[1] + 1, wz = hi[2] - lo[2] + 1;
   if (wx <= 0 || wy <= 0 || wz <= 0) return;  // block-uniform
   const int ncell = wx * wy * wz;
-  const Tri3 T = tri3(v, la.e, elem);
+  const Tri3 T = tri3(v, e, elem);
   const float far = 2.0f * la.cl;
-  unsigned long long* cells = table_cells(la, gen);
-  unsigned long long* keys = table_keys<3>(la, gen);
-  const int lane = (int)(threadIdx.x & 63u);
-  // finishes the ns gathered links; called block-uniformly, with ns read by
-  // every thread between two barriers
-  auto flush = [&](int ns) {
-    for (int q = (int)threadIdx.x; q < ns; q += NT) {
-      const int k = s_cell[q], l = s_dir[q];
-      const int i = lo[0] + k % wx, j = lo[1] + (k / wx) % wy, z = lo[2] + k / (wx * wy);
-      const float p1[3] = {(float)i * la.cl, (float)j * la.cl, (float)z * la.cl};
-      const float p2[3] = {((float)i - (float)d3_c(d3_pack(0), l)) * la.cl,
-                           ((float)j - (float)d3_c(d3_pack(1), l)) * la.cl,
-                           ((float)z - (float)d3_c(d3_pack(2), l)) * la.cl};
-      const float dd[3] = {p2[0] - p1[0], p2[1] - p1[1], p2[2] - p1[2]};
-      const float t = tri3_num(T, p1) / tri3_den(T, dd);
-      Hit h;
-      if (!(t < 0.0f || t > 1.0f) && tri3_finish(T, p1, dd, t, h)) {
-        const int slot = lt_claim(cells, la.cap, gen, (z * la.ny + j) * la.nx + i, &la.st->overflow);
-        if (slot >= 0) lt_offer_key(keys, (size_t)slot * K + (l - 1), gen, depth_key(h.depth, elem));
-      }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) s_n = 0;
-    __syncthreads();
+  const uint8_t* flags = dev_global(la.flags);
+  unsigned long long* cells = table_cells(la, tag);
+  unsigned long long* keys = table_keys<3>(la, tag);
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // link q of the pass at c0: bits 5.. the cell's place in the pass, 0-4 the direction
+  auto link_test = [&](int c0, unsigned q, int& cell, int& l, Hit& h) {
+    const int k = c0 + (int)(q >> 5);
+    l = (int)(q & 31u);
+    const int i = lo[0] + k % wx, j = lo[1] + (k / wx) % wy, z = lo[2] + k / (wx * wy);
+    cell = (z * la.ny + j) * la.nx + i;
+    const float p1[3] = {(float)i * la.cl, (float)j * la.cl, (float)z * la.cl};
+    const float p2[3] = {((float)i - (float)d3_c(d3_pack(0), l)) * la.cl,
+                         ((float)j - (float)d3_c(d3_pack(1), l)) * la.cl,
+                         ((float)z - (float)d3_c(d3_pack(2), l)) * la.cl};
+    return hit_tri3(T, p1, p2, h);
   };
-  if (threadIdx.x == 0) s_n = 0;
-  __syncthreads();
-  for (int c0 = 0; c0 < ncell; c0 += NT) {
-    const int k = c0 + (int)threadIdx.x;
-    bool near = false;
-    float fi = 0.0f, fj = 0.0f, fz = 0.0f, num = 0.0f;
-    if (k < ncell) {
-      const int i = lo[0] + k % wx, j = lo[1] + (k / wx) % wy, z = lo[2] + k / (wx * wy);
-      if (is_updated(la.flags[(z * la.ny + j) * la.nx + i])) {
-        fi = (float)i;
-        fj = (float)j;
-        fz = (float)z;
-        const float p1[3] = {fi * la.cl, fj * la.cl, fz * la.cl};
-        num = tri3_num(T, p1);
-        near = fabsf(num) <= far;
+  for (int c0 = 0; c0 < ncell; c0 += U * NT) {
+    unsigned may[U];
+    bool upd[U];
+#pragma unroll
+    for (int w = 0; w < U; w++) {  // both flags in flight
+      const int k = c0 + w * NT + tid;
+      upd[w] = false;
+      if (k < ncell) {
+        const int i = lo[0] + k % wx, j = lo[1] + (k / wx) % wy, z = lo[2] + k / (wx * wy);
+        upd[w] = is_updated(flags[(z * la.ny + j) * la.nx + i]);
       }
     }
-    const float p1[3] = {fi * la.cl, fj * la.cl, fz * la.cl};
+    int count = 0;
 #pragma unroll
-    for (int l = 1; l <= K; l++) {
-      bool keep = false;
-      if (near) {
-        const float p2[3] = {(fi - (float)d3_c(d3_pack(0), l)) * la.cl, (fj - (float)d3_c(d3_pack(1), l)) * la.cl,
-                             (fz - (float)d3_c(d3_pack(2), l)) * la.cl};
-        const float dd[3] = {p2[0] - p1[0], p2[1] - p1[1], p2[2] - p1[2]};
-        keep = tri3_t_may_pass(num, tri3_den(T, dd));
-      }
-      const unsigned long long m = __ballot(keep);
-      if (m) {
-        int base = 0;
-        if (lane == 0) base = atomicAdd(&s_n, __popcll(m));
-        base = __shfl(base, 0, 64);
-        if (keep) {
-          const int idx = base + __popcll(m & ((1ull << lane) - 1ull));
-          s_cell[idx] = k;
-          s_dir[idx] = (unsigned char)l;
+    for (int w = 0; w < U; w++) {
+      may[w] = 0;
+      if (upd[w]) {
+        const int k = c0 + w * NT + tid;
+        const float fi = (float)(lo[0] + k % wx), fj = (float)(lo[1] + (k / wx) % wy),
+                    fz = (float)(lo[2] + k / (wx * wy));
+        const float p1[3] = {fi * la.cl, fj * la.cl, fz * la.cl};
+        const float num = tri3_num(T, p1);
+        if (fabsf(num) <= far) {
+#pragma unroll
+          for (int l = 1; l <= K; l++) {
+            const float p2[3] = {(fi - (float)D3::cx(l)) * la.cl, (fj - (float)D3::cy(l)) * la.cl,
+                                 (fz - (float)D3::cz(l)) * la.cl};
+            const float dd[3] = {p2[0] - p1[0], p2[1] - p1[1], p2[2] - p1[2]};
+            if (tri3_t_may_pass(num, tri3_den(T, dd))) may[w] |= 1u << l;
+          }
         }
       }
-      // at most 4 * NT entries join between checks: finish the lists while
-      // that still fits
-      if (l % 4 == 0 || l == K) {
-        __syncthreads();
-        const int ns = s_n;
-        __syncthreads();  // read by all before any wave adds again
-        if (ns > kDet3Cap - 4 * NT) flush(ns);
-      }
+      count += __popc(may[w]);
     }
+    // block-wide prefix sum of the counts
+    int before = count;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int o = __shfl_up(before, off, 64);
+      if (lane >= off) before += o;
+    }
+    if (lane == 63) s_wave[wave] = before;
+    __syncthreads();
+    before -= count;
+    int total = 0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      before += w < wave ? s_wave[w] : 0;
+      total += s_wave[w];
+    }
+    for (int base = 0; base < total; base += kDet3Cap) {
+      if (tid == 0) s_nhit = 0;
+      int at = before - base;
+#pragma unroll
+      for (int w = 0; w < U; w++)
+        for (unsigned m = may[w]; m; m &= m - 1, at++)
+          if (at >= 0 && at < kDet3Cap)
+            s_may[at] = (unsigned short)(((w * NT + tid) << 5) | (__ffs((int)m) - 1));
+      __syncthreads();
+      const int ns = min(total - base, kDet3Cap);
+      for (int q0 = 0; q0 < ns; q0 += NT) {
+        const int q = q0 + tid;
+        int cell, l;
+        Hit h;
+        const bool hit = q < ns && link_test(c0, s_may[q], cell, l, h);
+        const unsigned long long m = __ballot(hit);
+        if (m) {
+          int pos = 0;
+          if (lane == 0) pos = atomicAdd(&s_nhit, (int)__popcll(m));
+          pos = __shfl(pos, 0, 64);
+          if (hit) s_hit[pos + (int)__popcll(m & ((1ull << lane) - 1ull))] = s_may[q];
+        }
+      }
+      __syncthreads();
+      const int nh = s_nhit;
+      for (int q = tid; q < nh; q += NT) {
+        int cell, l;
+        Hit h;
+        link_test(c0, s_hit[q], cell, l, h);
+        const int slot = lt_claim(cells, la.cap, tag, cell, &la.st->overflow);
+        if (slot >= 0) lt_offer_key(keys, (size_t)slot * K + (l - 1), tag, depth_key(h.depth, elem));
+      }
+      __syncthreads();  // the lists and counters are free again
+    }
+    if (total == 0) __syncthreads();  // s_wave is read before the next pass writes it
   }
-  __syncthreads();
-  const int ns = s_n;
-  if (ns > 0) flush(ns);
 }
 
-// Detection block of a batch (blockDim = kDetectLanes<3> = 256): 2D packs
-// blockDim / kDetectLanes<2> elements per block (32 lanes per segment: about
-// 5 tasks each, fewer waves in flight for the same work than 64), 3D takes one
-// element per block.
-static_assert(kDetectLanes<3> == 256, "build_links_block3 assumes 256-thread blocks");
-template <int DIM>
+// Detection block of 256 threads: 2D takes blockDim / kRow elements (ROWS) or
+// (element, direction) pairs, 3D one element.
+template <int DIM, bool ROWS>
 __device__ __forceinline__ void detect_block(const LinkArgs& la, long long block, unsigned tag, const float* v) {
-  if constexpr (DIM == 2)
-    build_links_block2<kDetectLanes<2>>(la, block, tag, v);
-  else
+  if constexpr (DIM == 3)
     build_links_block3(la, block, tag, v);
+  else if constexpr (ROWS)
+    build_links_rows2(la, block, tag, v);
+  else
+    build_links_pairs2(la, block, tag, v);
 }
 
 }  // namespace ff

@@ -611,6 +611,18 @@ struct h16u {
   unsigned short bits;
 };
 
+// The units that instantiate every tile shape are compiled once per storage
+// format (FF_TU_STORAGE, an FF_STORAGE_* value); the one for format 0 also
+// holds their host code.
+#ifdef FF_TU_STORAGE
+template <int> struct tu_type;
+template <> struct tu_type<0> { using type = float; };
+template <> struct tu_type<1> { using type = __half; };
+template <> struct tu_type<2> { using type = __hip_bfloat16; };
+template <> struct tu_type<3> { using type = h16u; };
+using tu_storage = tu_type<FF_TU_STORAGE>::type;
+#endif
+
 // Moment loads and stores by storage type: p points at the cell's value in
 // plane k; `plane` is the plane stride in elements (used by the split
 // velocity of h16u).

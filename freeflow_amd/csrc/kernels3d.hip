@@ -100,7 +100,7 @@ static void step3d_variant(Domain& d, const S* i, S* o, const LinkArgs& la, cons
 }
 
 template <typename S>
-static int step3d_typed(Domain& d, const void* in, void* out, const LinkArgs& la, const FinalArgs& fa, bool wave) {
+int step3d_typed(Domain& d, const void* in, void* out, const LinkArgs& la, const FinalArgs& fa, bool wave) {
   const bool per = d.options & FF_OPT_PERIODIC, fast = d.options & FF_OPT_FAST_MATH;
   if (per && fast) step3d_variant<S, true, true>(d, (const S*)in, (S*)out, la, fa, wave);
   else if (per) step3d_variant<S, true, false>(d, (const S*)in, (S*)out, la, fa, wave);
@@ -109,6 +109,29 @@ static int step3d_typed(Domain& d, const void* in, void* out, const LinkArgs& la
   FF_HIP(hipGetLastError());
   return FF_OK;
 }
+
+template <typename S>
+int bulk3d_typed(Domain& d, const void* in, void* out) {
+  const bool per = d.options & FF_OPT_PERIODIC, fast = d.options & FF_OPT_FAST_MATH;
+  if (per && fast) bulk3d_variant<S, true, true>(d, (const S*)in, (S*)out);
+  else if (per) bulk3d_variant<S, true, false>(d, (const S*)in, (S*)out);
+  else if (fast) bulk3d_variant<S, false, true>(d, (const S*)in, (S*)out);
+  else bulk3d_variant<S, false, false>(d, (const S*)in, (S*)out);
+  FF_HIP(hipGetLastError());
+  return FF_OK;
+}
+
+template int step3d_typed<tu_storage>(Domain&, const void*, void*, const LinkArgs&, const FinalArgs&, bool);
+template int bulk3d_typed<tu_storage>(Domain&, const void*, void*);
+
+#if FF_TU_STORAGE == 0
+#define FF_ELSEWHERE(S)                                                                                          \
+  extern template int step3d_typed<S>(Domain&, const void*, void*, const LinkArgs&, const FinalArgs&, bool); \
+  extern template int bulk3d_typed<S>(Domain&, const void*, void*);
+FF_ELSEWHERE(__half)
+FF_ELSEWHERE(__hip_bfloat16)
+FF_ELSEWHERE(h16u)
+#undef FF_ELSEWHERE
 
 int launch_step_stream3d(Domain& d, const void* in, void* out, const LinkArgs& la, FinalArgs fa, bool wave) {
   switch (d.storage) {
@@ -119,17 +142,6 @@ int launch_step_stream3d(Domain& d, const void* in, void* out, const LinkArgs& l
   }
 }
 
-template <typename S>
-static int bulk3d_typed(Domain& d, const void* in, void* out) {
-  const bool per = d.options & FF_OPT_PERIODIC, fast = d.options & FF_OPT_FAST_MATH;
-  if (per && fast) bulk3d_variant<S, true, true>(d, (const S*)in, (S*)out);
-  else if (per) bulk3d_variant<S, true, false>(d, (const S*)in, (S*)out);
-  else if (fast) bulk3d_variant<S, false, true>(d, (const S*)in, (S*)out);
-  else bulk3d_variant<S, false, false>(d, (const S*)in, (S*)out);
-  FF_HIP(hipGetLastError());
-  return FF_OK;
-}
-
 int launch_bulk3d(Domain& d, const void* in, void* out) {
   switch (d.storage) {
     case FF_STORAGE_F32: return bulk3d_typed<float>(d, in, out);
@@ -138,5 +150,7 @@ int launch_bulk3d(Domain& d, const void* in, void* out) {
     default: return bulk3d_typed<__hip_bfloat16>(d, in, out);
   }
 }
+
+#endif
 
 }  // namespace ff

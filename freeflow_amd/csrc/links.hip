@@ -14,8 +14,8 @@
 // Forces: the reference scatters every link force to the element's vertices
 // with float atomicAdd (SolidGeometryProxy_Device.cuh:184-194, 401-421), whose
 // order is nondeterministic.  Here each link force is stored with its link;
-// each element then sums its own links in a fixed order (one wave per
-// element), and the finish phase sums elements into vertices (CSR order) and
+// each element then sums its own links in a fixed order (a row of lanes per
+// segment, a block per triangle), and the finish phase sums elements into vertices (CSR order) and
 // bodies, all in FP64.  Results do not depend on scheduling.
 //
 // A step with a boundary is two launches (three when the links must be
@@ -46,13 +46,13 @@ namespace ff {
 // Links of the current step under the current tag and vertex buffer.
 template <int DIM>
 __global__ void __launch_bounds__(256) k_links_build(LinkArgs la) {
-  build_links_pairs<DIM>(la, blockIdx.x, step_tag(la), la.v[step_gen(la) & 1]);
+  detect_block<DIM, false>(la, blockIdx.x, step_tag(la), la.v[step_gen(la) & 1]);
 }
 
 // Links of the current step of a domain stepped on its own (a batch detects
 // its pending members with kb_detect).
 int launch_detect(Domain& d, const LinkArgs& la) {
-  const unsigned g = (unsigned)detect_blocks(d, 256, false);
+  const unsigned g = (unsigned)detect_blocks(d, false);
   if (g > 0) {
     if (d.dim == 2) k_links_build<2><<<g, 256, 0, d.stream>>>(la);
     else k_links_build<3><<<g, 256, 0, d.stream>>>(la);
@@ -79,12 +79,12 @@ __global__ void __launch_bounds__(FB) k_step_finish(LinkArgs la, FinalArgs fa, i
   else finish_last_body<DIM, FB>(la, fa, fa.fin_gen, false);
 }
 
-// Detection blocks of `nt` threads: batched, one element per kDetectLanes
-// lanes; otherwise one (element, direction) pair per 16 lanes.
-int detect_blocks(const Domain& d, int nt, bool batched) {
-  if (!batched) return (int)(((long long)d.ne * (d.q - 1) + nt / 16 - 1) / (nt / 16));
-  const long long per = std::max(1, nt / (d.dim == 2 ? kDetectLanes<2> : kDetectLanes<3>));
-  return (int)(((long long)d.ne + per - 1) / per);
+// Detection blocks of 256 threads (detect_block).
+int detect_blocks(const Domain& d, bool batched) {
+  if (d.dim == 3) return d.ne;
+  constexpr int per = 256 / kRow;
+  const int n = batched ? d.ne : d.ne * (d.q - 1);  // at most 65536 elements
+  return (n + per - 1) / per;
 }
 
 // Copy-back blocks of the sums launch and boundary-cell blocks of the stream
@@ -113,7 +113,7 @@ int launch_step_sums(Domain& d, const LinkArgs& la, void* out, bool detect_next)
   constexpr int FB = kSumBlock;
   const FinalArgs fa = make_final_args(d, out, d.vbuf[0], d.vbuf[1], d.ubuf[0], d.ubuf[1], nullptr);
   const unsigned grid =
-      (unsigned)(elem_blocks(d.ne) + fa.outlet_blocks + fa.copy_blocks + (detect_next ? detect_blocks(d, kSumBlock, false) : 0));
+      (unsigned)(elem_blocks(d.dim, d.ne) + fa.outlet_blocks + fa.copy_blocks + (detect_next ? detect_blocks(d, false) : 0));
 #define FF_SUM(DIM, S) k_step_sums<DIM, S, FB><<<grid, FB, 0, d.stream>>>(la, fa, out)
   if (d.dim == 2) {
     if (d.storage == FF_STORAGE_F32) FF_SUM(2, float);

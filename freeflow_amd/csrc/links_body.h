@@ -255,10 +255,14 @@ struct FinalArgs {
   unsigned fin_gen;
 };
 
-// Block size of the element-sum launch (2D and 3D) and elements per block
-// (one per wave).
-constexpr int kSumBlock = 256, kElemPerBlock = kSumBlock / 64;
-__host__ __device__ inline int elem_blocks(int ne) { return (ne + kElemPerBlock - 1) / kElemPerBlock; }
+// Block size of the element-sum launch, and blocks for the sums of `ne`
+// elements: kRow lanes per segment in 2D, a block per triangle in 3D (see
+// elem_sum2 / elem_sum3).
+constexpr int kSumBlock = 256;
+__host__ __device__ inline int elem_blocks(int dim, int ne) {
+  constexpr int per = kSumBlock / kRow;
+  return dim == 2 ? (ne + per - 1) / per : ne;
+}
 
 // Host: the FinalArgs of a domain (outlets written into `out`, next-step
 // kinematics into vn/un, per-vertex forces optionally added to proxy_forces).
@@ -266,7 +270,6 @@ FinalArgs make_final_args(Domain& d, void* out, float* vn0, float* vn1, float* u
 // Host: grid sizes of the boundary-cell and copy-back parts of a step.
 int boundary_cell_blocks(const Domain& d, int span);
 int copyback_blocks(const Domain& d, int fb, int per_thread);
-int detect_blocks(const Domain& d, int nt, bool batched);
 
 // Travelling wave along the body axis:
 //   y = y_rest + A s sin(theta), v_y = -2 pi f A s cos(theta),
@@ -339,166 +342,248 @@ __device__ __forceinline__ void wave_block_body(const LinkArgs& la, const FinalA
 template <int DIM, bool BATCHED>
 __device__ __forceinline__ void detect_next_body(const LinkArgs& la, int blk) {
   const unsigned gen = step_gen(la);
-  if constexpr (BATCHED)
-    detect_block<DIM>(la, (long long)blk, step_tag(la) + 1u, la.v[(gen + 1u) & 1u]);
-  else
-    build_links_pairs<DIM>(la, (long long)blk, step_tag(la) + 1u, la.v[(gen + 1u) & 1u]);
+  detect_block<DIM, BATCHED>(la, (long long)blk, step_tag(la) + 1u, la.v[(gen + 1u) & 1u]);
+}
+
+// ---------------------------------------------------------------- element sums
+// v of lane + N of the same DPP row (16 lanes), 0 beyond its end.
+template <int N>
+__device__ __forceinline__ double row_down(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, 0x100 | N, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), 0x100 | N, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+// Lane 0 of every row ends with the row's sums (a fixed tree).
+template <int M>
+__device__ __forceinline__ void row_sums(double* a) {
+#pragma unroll
+  for (int k = 0; k < M; k++) a[k] += row_down<8>(a[k]);
+#pragma unroll
+  for (int k = 0; k < M; k++) a[k] += row_down<4>(a[k]);
+#pragma unroll
+  for (int k = 0; k < M; k++) a[k] += row_down<2>(a[k]);
+#pragma unroll
+  for (int k = 0; k < M; k++) a[k] += row_down<1>(a[k]);
+}
+
+// Bit l set: direction l + 1 of the slot holds a key of this generation that
+// names element `etag` (the winner of the link).
+template <int DIM>
+__device__ __forceinline__ unsigned links_of_element(const unsigned long long* keys, int slot, unsigned tag,
+                                                     unsigned etag) {
+  constexpr int K = DIM == 2 ? 8 : 26;
+  // a row of keys is K * 8 bytes, a multiple of 16, in a 256-byte aligned table
+  const ulonglong2* row = reinterpret_cast<const ulonglong2*>(keys + (size_t)slot * K);
+  unsigned m = 0;
+#pragma unroll
+  for (int l = 0; l < K; l += 2) {
+    const ulonglong2 w = row[l / 2];
+    if ((unsigned)(w.x >> 32) == tag && (~(unsigned)w.x & 0xFFFFu) == etag) m |= 1u << l;
+    if ((unsigned)(w.y >> 32) == tag && (~(unsigned)w.y & 0xFFFFu) == etag) m |= 2u << l;
+  }
+  return m;
+}
+
+// Sum of one segment's links by a row of kRow lanes: each lane takes up to two
+// window cells per pass (its own table probes and key rows in flight
+// together), then the links of those cells that name this element, in
+// direction order; a fixed tree folds the lanes.  The pass is a chain of
+// dependent loads (vertices -> table -> keys -> links) at every step's end, and
+// with many domains it is bound by instruction issue: one (cell, direction)
+// task per lane loaded every link's force and geometry before knowing whose
+// it was, and folded one element per wave.
+__device__ __forceinline__ void elem_sum2(const LinkArgs& la, const FinalArgs& fa, int elem, int lane) {
+  constexpr int K = 8, STRIDE = elem_stride_v<2>, U = 2;
+  const unsigned gen = step_gen(la), tag = step_tag(la);
+  const float* v = dev_global(la.v[gen & 1]);
+  const float* u = dev_global(la.u[gen & 1]);
+  const u32x2 ends = load2(dev_global(la.e) + 2 * (size_t)elem);
+  const int body = fa.elem_body ? dev_global(fa.elem_body)[elem] : 0;
+  const f32x2 pa = load2(v + 2 * (size_t)ends.x), pb = load2(v + 2 * (size_t)ends.y);
+  const f32x2 ua = load2(u + 2 * (size_t)ends.x), ub = load2(u + 2 * (size_t)ends.y);
+  const double rx = dev_global(fa.body_ref)[2 * body], ry = dev_global(fa.body_ref)[2 * body + 1];
+  const int n[2] = {la.nx, la.ny};
+  int lo[2], hi[2];
+  seg_window(pa, pb, la.cl, n, lo, hi);
+  const int wx = hi[0] - lo[0] + 1, wy = hi[1] - lo[1] + 1;
+  const int ncell = (wx > 0 && wy > 0) ? wx * wy : 0;
+  double acc[STRIDE];
+#pragma unroll
+  for (int a = 0; a < STRIDE; a++) acc[a] = 0.0;
+  const unsigned etag = (unsigned)elem & 0xFFFFu;
+  const uint8_t* flags = dev_global(la.flags);
+  const unsigned long long* cells = table_cells(la, tag);
+  const unsigned long long* keys = table_keys<2>(la, tag);
+  const float* lf = dev_global(la.lf);
+  const float* lb = dev_global(la.lb);
+  const float* lh = dev_global(la.lh);
+  for (int k0 = lane; k0 < ncell; k0 += kRow * U) {
+    int cell[U];
+    unsigned home[U];
+    unsigned long long cur[U];
+    bool upd[U];
+#pragma unroll
+    for (int w = 0; w < U; w++) {
+      const int k = k0 + w * kRow;
+      upd[w] = false;
+      if (k < ncell) {
+        const int j = k / wx;
+        cell[w] = (lo[1] + j) * la.nx + lo[0] + (k - j * wx);
+        home[w] = lt_home(la.cap, cell[w]);
+        cur[w] = cells[home[w]];
+        upd[w] = is_updated(flags[cell[w]]);
+      }
+    }
+    int slot[U];
+#pragma unroll
+    for (int w = 0; w < U; w++) slot[w] = upd[w] ? lt_resolve(cells, la.cap, tag, cell[w], home[w], cur[w]) : -1;
+    unsigned m = 0;
+#pragma unroll
+    for (int w = 0; w < U; w++)
+      if (slot[w] >= 0) m |= links_of_element<2>(keys, slot[w], tag, etag) << (w * K);
+    while (m) {  // two links at a time
+      size_t li[2];
+      f32x2 F[2], B[2], H[2];
+      bool use[2];
+#pragma unroll
+      for (int w = 0; w < 2; w++) {
+        use[w] = m != 0;
+        if (use[w]) {
+          const int b = __ffs((int)m) - 1;
+          m &= m - 1;
+          li[w] = 2 * ((size_t)(b < K ? slot[0] : slot[1]) * K + (b & (K - 1)));
+          F[w] = load2(lf + li[w]);
+          B[w] = load2(lb + li[w]);
+          H[w] = load2(lh + li[w]);
+        }
+      }
+#pragma unroll
+      for (int w = 0; w < 2; w++) {
+        if (!use[w] || B[w].x == kLinkUnused) continue;
+        acc[0] += (double)(F[w].x * B[w].x);  // addForceAt products
+        acc[1] += (double)(F[w].y * B[w].x);
+        acc[2] += (double)(F[w].x * B[w].y);
+        acc[3] += (double)(F[w].y * B[w].y);
+        acc[4] += (double)F[w].x;
+        acc[5] += (double)F[w].y;
+        acc[6] += ((double)H[w].x - rx) * (double)F[w].y - ((double)H[w].y - ry) * (double)F[w].x;
+      }
+    }
+  }
+  row_sums<STRIDE - 1>(acc);
+  if (lane == 0) {
+    // the element's power: its vertex shares against the velocities the step used
+    acc[STRIDE - 1] =
+        -(acc[0] * (double)ua.x) - acc[1] * (double)ua.y - acc[2] * (double)ub.x - acc[3] * (double)ub.y;
+    double2* row = reinterpret_cast<double2*>(dev_global(fa.elem_acc) + (size_t)elem * STRIDE);
+#pragma unroll
+    for (int a = 0; a < STRIDE; a += 2) row[a / 2] = make_double2(acc[a], acc[a + 1]);
+  }
+}
+
+// Sum of one triangle's links by a block of kSumBlock threads: a window of
+// some 7^3 cells, one cell per thread and pass, its 26 keys read as one row.
+// One wave per triangle walked the same window in six passes of (cell,
+// direction) tasks, a serial chain of some 150 loads that set the launch's
+// time (76 us for the 320 triangles of a sphere in a 160x96x96 domain).
+// The rows of 16 lanes are folded by a fixed tree, their sums in row order.
+__device__ __forceinline__ void elem_sum3(const LinkArgs& la, const FinalArgs& fa, int elem) {
+  constexpr int K = 26, STRIDE = elem_stride_v<3>, M = STRIDE - 1, NROW = kSumBlock / kRow;
+  static_assert(M <= kRow, "one lane of a row per sum");
+  __shared__ double s_part[NROW][kRow];
+  const unsigned gen = step_gen(la), tag = step_tag(la);
+  const float* v = dev_global(la.v[gen & 1]);
+  const int n[3] = {la.nx, la.ny, la.nz};
+  int lo[3], hi[3];
+  elem_window<3>(v, dev_global(la.e), elem, la.cl, n, lo, hi);
+  const int wx = hi[0] - lo[0] + 1, wy = hi[1] - lo[1] + 1, wz = hi[2] - lo[2] + 1;
+  const int ncell = (wx > 0 && wy > 0 && wz > 0) ? wx * wy * wz : 0;
+  const int body = fa.elem_body ? dev_global(fa.elem_body)[elem] : 0;
+  double ref[3];
+#pragma unroll
+  for (int c = 0; c < 3; c++) ref[c] = dev_global(fa.body_ref)[body * 3 + c];
+  double acc[M];
+#pragma unroll
+  for (int a = 0; a < M; a++) acc[a] = 0.0;
+  const unsigned etag = (unsigned)elem & 0xFFFFu;
+  const uint8_t* flags = dev_global(la.flags);
+  const unsigned long long* cells = table_cells(la, tag);
+  const unsigned long long* keys = table_keys<3>(la, tag);
+  const float* lf = dev_global(la.lf);
+  const float* lb = dev_global(la.lb);
+  const float* lh = dev_global(la.lh);
+  for (int k = (int)threadIdx.x; k < ncell; k += kSumBlock) {
+    const int i = lo[0] + k % wx, j = lo[1] + (k / wx) % wy, z = lo[2] + k / (wx * wy);
+    const int cell = (z * la.ny + j) * la.nx + i;
+    const unsigned home = lt_home(la.cap, cell);
+    const unsigned long long cur = cells[home];
+    if (!is_updated(flags[cell])) continue;
+    const int slot = lt_resolve(cells, la.cap, tag, cell, home, cur);
+    if (slot < 0) continue;
+    for (unsigned m = links_of_element<3>(keys, slot, tag, etag); m; m &= m - 1) {
+      const size_t li = ((size_t)slot * K + (__ffs((int)m) - 1)) * 3;
+      float F[3], B[3], H[3];
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        F[c] = lf[li + c];
+        B[c] = lb[li + c];
+        H[c] = lh[li + c];
+      }
+      if (B[0] == kLinkUnused) continue;
+#pragma unroll
+      for (int jv = 0; jv < 3; jv++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) acc[jv * 3 + c] += (double)(F[c] * B[jv]);  // addForceAt products
+      double r[3];
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        acc[9 + c] += (double)F[c];
+        r[c] = (double)H[c] - ref[c];
+      }
+      acc[12] += r[1] * (double)F[2] - r[2] * (double)F[1];
+      acc[13] += r[2] * (double)F[0] - r[0] * (double)F[2];
+      acc[14] += r[0] * (double)F[1] - r[1] * (double)F[0];
+    }
+  }
+  row_sums<M>(acc);
+  const int row = (int)threadIdx.x / kRow, lane = (int)threadIdx.x % kRow;
+  if (lane == 0) {
+#pragma unroll
+    for (int a = 0; a < M; a++) s_part[row][a] = acc[a];
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < kRow) {
+    double t = 0.0;
+    if (lane < M) {
+#pragma unroll
+      for (int r = 0; r < NROW; r++) t += s_part[r][lane];
+    }
+    // the element's power: its vertex shares against the velocities the step used
+    double pw = 0.0;
+    if (lane < 9) {
+      const size_t vid = dev_global(la.e)[(size_t)elem * 3 + lane / 3];
+      pw = -t * (double)dev_global(la.u[gen & 1])[vid * 3 + lane % 3];
+    }
+    row_sums<1>(&pw);
+    double* out = dev_global(fa.elem_acc) + (size_t)elem * STRIDE;
+    if (lane < M) out[lane] = t;
+    if (lane == 0) out[STRIDE - 1] = pw;
+  }
 }
 
 // Second launch of a boundary step, kSumBlock threads per block.  The first
-// ceil(ne / kElemPerBlock) blocks sum links per element, one element per
-// wave: each sums its own links (fixed order, FP64) into elem_acc.  Then
-// outlet blocks: outlet cells of the freshly written buffer
+// elem_blocks blocks sum links per element (fixed order, FP64) into elem_acc.
+// Then outlet blocks: outlet cells of the freshly written buffer
 // (mrApplyOutlet2DKernel / mrApplyOutlet3DKernel; a neighbour that is a
 // boundary cell is read from its side-buffer row, which the copy-back of this
 // launch writes).  Then copy-back blocks: boundary-cell rows into the output.
 // Any further blocks detect the next step's links.
-// Sum of one element's links by one wave (lane = lane index, sl = 64 ints of
-// LDS for the wave): window cells are resolved 64 at a time, then every lane
-// takes (cell, direction) tasks; a fixed shuffle tree folds the FP64 sums.
-// PAIR: a lane's 2D tasks two at a time (a domain stepped on its own, where
-// the launch's latency is the slowest wave's); the sums do not depend on it.
-template <int DIM, bool PAIR>
-__device__ __forceinline__ void elem_sum_wave(const LinkArgs& la, const FinalArgs& fa, int elem, int lane, int* sl) {
-  constexpr int K = DIM == 2 ? 8 : 26;
-  constexpr int NT = DIM == 2 ? 1 : 3;
-  constexpr int STRIDE = elem_stride_v<DIM>;
-  const unsigned gen = step_gen(la);
-  const unsigned tag = step_tag(la);
-  const float* v = la.v[gen & 1];
-  const int n[3] = {la.nx, la.ny, la.nz};
-  int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-  elem_window<DIM>(v, la.e, elem, la.cl, n, lo, hi);
-  const int wx = hi[0] - lo[0] + 1, wy = hi[1] - lo[1] + 1, wz = DIM == 3 ? hi[2] - lo[2] + 1 : 1;
-  const int ncell = (wx > 0 && wy > 0 && wz > 0) ? wx * wy * wz : 0;
-  const int b = fa.elem_body ? fa.elem_body[elem] : 0;
-  double ref[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-  for (int c = 0; c < DIM; c++) ref[c] = fa.body_ref[b * DIM + c];
-  double acc[STRIDE];
-#pragma unroll
-  for (int a = 0; a < STRIDE; a++) acc[a] = 0.0;
-  const uint32_t etag = (uint32_t)(uint16_t)elem;
-  const unsigned long long* cells = table_cells(la, tag);
-  const unsigned long long* keys = table_keys<DIM>(la, tag);
-  for (int c0 = 0; c0 < ncell; c0 += 64) {
-    const int chunk = min(64, ncell - c0);
-    if (lane < chunk) {
-      const int kk = c0 + lane;
-      const int i = lo[0] + kk % wx, j = lo[1] + (kk / wx) % wy, z = DIM == 3 ? lo[2] + kk / (wx * wy) : 0;
-      const int cell = (z * la.ny + j) * la.nx + i;
-      // the flag and the table probe are independent loads: issue both
-      const int found = lt_find(cells, la.cap, tag, cell);
-      sl[lane] = is_updated(la.flags[cell]) ? found : -1;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // 2D: every load of a task issued before any test, and with PAIR a
-    // lane's tasks two at a time (the loads of both overlap), added in task
-    // order, so the FP64 sums are those of a one-at-a-time loop.  3D: one task at a time,
-    // and a link's force and geometry are loaded only once its key names
-    // this element (a 3D window's cells carry mostly other elements' links;
-    // loading them all doubled the batched 3D sums launch).
-    constexpr int U = DIM == 2 && PAIR ? 2 : 1;
-    constexpr bool EARLY = DIM == 2;
-    for (int t0 = lane; t0 < K * chunk; t0 += 64 * U) {
-      bool use[U];
-      uint32_t key[U];
-      size_t lis[U];
-      float F[U][DIM], B[U][DIM], H[U][DIM];
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int task = t0 + 64 * u;
-        const int k = task % chunk, l = task / chunk;
-        const int slot = task < K * chunk ? sl[k] : -1;
-        use[u] = slot >= 0;
-        key[u] = 0xFFFFFFFFu;
-        lis[u] = 0;
-        if (use[u]) {  // every load of the link lies inside the slot's rows
-          const size_t li = (size_t)slot * K + l;
-          lis[u] = li;
-          key[u] = lt_key(keys, li, tag);
-          if constexpr (EARLY) {
-#pragma unroll
-            for (int c = 0; c < DIM; c++) {
-              F[u][c] = la.lf[li * DIM + c];
-              B[u][c] = la.lb[li * DIM + c];
-              H[u][c] = la.lh[li * DIM + c];
-            }
-          }
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        if (!use[u] || key[u] == 0xFFFFFFFFu || (key[u] & 0xFFFFu) != etag) continue;
-        if constexpr (!EARLY) {
-          const size_t li = lis[u];
-          if (la.lb[li * DIM] == kLinkUnused) continue;
-#pragma unroll
-          for (int c = 0; c < DIM; c++) {
-            F[u][c] = la.lf[li * DIM + c];
-            B[u][c] = la.lb[li * DIM + c];
-            H[u][c] = la.lh[li * DIM + c];
-          }
-        }
-        if (B[u][0] == kLinkUnused) continue;
-#pragma unroll
-        for (int jv = 0; jv < DIM; jv++) {
-          const float bj = B[u][jv];
-#pragma unroll
-          for (int c = 0; c < DIM; c++) acc[jv * DIM + c] += (double)(F[u][c] * bj);  // addForceAt products
-        }
-#pragma unroll
-        for (int c = 0; c < DIM; c++) acc[DIM * DIM + c] += (double)F[u][c];
-        double r[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-        for (int c = 0; c < DIM; c++) r[c] = (double)H[u][c] - ref[c];
-        if constexpr (DIM == 2) {
-          acc[DIM * DIM + DIM] += r[0] * (double)F[u][1] - r[1] * (double)F[u][0];
-        } else {
-          acc[DIM * DIM + DIM + 0] += r[1] * (double)F[u][2] - r[2] * (double)F[u][1];
-          acc[DIM * DIM + DIM + 1] += r[2] * (double)F[u][0] - r[0] * (double)F[u][2];
-          acc[DIM * DIM + DIM + 2] += r[0] * (double)F[u][1] - r[1] * (double)F[u][0];
-        }
-      }
-    }
-    // the next chunk overwrites sl[] only after every lane's reads above
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  }
-  // fixed shuffle tree over the wave's 64 lanes
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-    for (int a = 0; a < STRIDE; a++) acc[a] += __shfl_down(acc[a], off, 64);
-  }
-  if (lane == 0) {
-    // the element's power: its vertex shares against the velocities the step used
-    const float* u = la.u[gen & 1];
-    double pw = 0.0;
-#pragma unroll
-    for (int jv = 0; jv < DIM; jv++) {
-      const size_t vid = la.e[(size_t)elem * DIM + jv];
-#pragma unroll
-      for (int c = 0; c < DIM; c++) pw -= acc[jv * DIM + c] * (double)u[vid * DIM + c];
-    }
-    acc[STRIDE - 1] = pw;
-#pragma unroll
-    for (int a = 0; a < STRIDE; a++) fa.elem_acc[(size_t)elem * STRIDE + a] = acc[a];
-  }
-}
-
-
 template <int DIM, typename S, int FB, bool BATCHED>
 __device__ __forceinline__ void elem_sums_body(const LinkArgs& la, const FinalArgs& fa, int blk, void* out) {
-  static_assert(FB == kSumBlock, "element sums run one element per wave of a kSumBlock block");
-  constexpr int K = DIM == 2 ? 8 : 26;
-  constexpr int NT = DIM == 2 ? 1 : 3;
+  static_assert(FB == kSumBlock, "element sums and detection are written for kSumBlock threads");
   constexpr int NM = DIM == 2 ? 6 : 10;
-  constexpr int STRIDE = elem_stride_v<DIM>;
-  const int neb = elem_blocks(la.ne);
+  const int neb = elem_blocks(DIM, la.ne);
   if (blk >= neb + fa.outlet_blocks + fa.copy_blocks) {
     detect_next_body<DIM, BATCHED>(la, blk - neb - fa.outlet_blocks - fa.copy_blocks);
     return;
@@ -541,10 +626,12 @@ __device__ __forceinline__ void elem_sums_body(const LinkArgs& la, const FinalAr
     Store<S>::template store<DIM>(buf + c.pcomp * la.plane + c.cell, c.pcomp, up * up, la.plane);
     return;
   }
-  __shared__ int s_slot[kElemPerBlock][64];
-  const int wv = threadIdx.x >> 6;
-  const int elem = blk * kElemPerBlock + wv;
-  if (elem < la.ne) elem_sum_wave<DIM, !BATCHED>(la, fa, elem, threadIdx.x & 63, s_slot[wv]);
+  if constexpr (DIM == 2) {
+    const int elem = blk * (FB / kRow) + (int)threadIdx.x / kRow;
+    if (elem < la.ne) elem_sum2(la, fa, elem, (int)threadIdx.x % kRow);
+  } else {
+    elem_sum3(la, fa, blk);
+  }
 }
 
 // Vertex blocks sum their incident element shares in CSR order (the
