@@ -7,6 +7,7 @@
 //
 //   kb_step      boundary cells (into side-buffer rows), next-step wave
 //                kinematics and the stream-collide tiles of every domain
+//                (kb_sep3d beside it if members step with the separable form)
 //   kb_sums      per-element FP64 force sums, outlet cells, the
 //                boundary-cell copy-back and the next step's link detection
 //                of every domain
@@ -37,6 +38,7 @@
 #include "ff_internal.h"
 #include "geometry.h"
 #include "links_body.h"
+#include "separable3d.h"
 #include "stencil.h"
 
 namespace ff {
@@ -51,6 +53,7 @@ struct DomDev {
   int nvb;           // vertex blocks of the finish phase
   int ndet;          // next-step detection blocks of the element-sum phase
   int boundary;
+  int chunks;        // z chunks of the separable 3D form, 0: tiles
   int* bflag;        // the batch's overflow flag (set when this domain's table overflowed)
 };
 
@@ -69,7 +72,7 @@ struct Batch {
   size_t map_cap = 0;
   unsigned* d_steps = nullptr;
   size_t steps_cap = 0;
-  int n_bc = 0, n_wave = 0, n_bulk = 0, n_es = 0, n_fin = 0;
+  int n_bc = 0, n_wave = 0, n_bulk = 0, n_sep = 0, n_es = 0, n_fin = 0;
   int* d_flag = nullptr;  // set by a replay whose detection overflowed a member's link table
   // pending detections (members whose links were not detected ahead): pinned
   // staging and its device copy, reused or regrown only once the copy and the
@@ -246,13 +249,16 @@ static void launch_tail(Batch& b, const int2* map_sums, const int2* map_fin) {
   if (b.n_fin > 0) kb_finish<DIM, 256><<<b.n_fin, 256, 0, b.stream>>>(b.d_doms, map_fin);
 }
 
+void launch_sep(Batch& b);
+
 template <typename S>
 void launch_step_typed(Batch& b, int tile) {
   const int n_stream = b.n_bc + b.n_wave + b.n_bulk;
   const int2* map_stream = b.d_map;
-  const int2* map_sums = map_stream + n_stream;
+  const int2* map_sums = map_stream + n_stream + b.n_sep;
   const int2* map_fin = map_sums + b.n_es;
   launch_stream_batch<S>(b, tile, map_stream, n_stream, b.n_bc, b.n_wave);
+  if constexpr (std::is_same<S, float>::value) launch_sep(b);
   if (b.dim == 2) launch_tail<2, S>(b, map_sums, map_fin);
   else launch_tail<3, S>(b, map_sums, map_fin);
 }
@@ -301,6 +307,27 @@ static void launch_step(Batch& b, int tile) {
   else launch_step_typed<__hip_bfloat16>(b, tile);
 }
 
+// Members that step with the separable 3D form (no body, so nothing else of
+// the stream launch is theirs).
+template <bool PERIODIC>
+__global__ void __launch_bounds__(kSepThreads, 5)
+    kb_sep3d(const DomDev* __restrict__ doms, const int2* __restrict__ map) {
+  const int2 m = map[blockIdx.x];
+  if (m.x < 0) return;  // padding of the XCD-aware tile order
+  const DomDev* D = doms + m.x;
+  const unsigned p = *D->step & 1u;
+  const LinkArgs& la = D->la;
+  sep3d_tile<PERIODIC>(dev_global((const float*)D->mom[p]), dev_global((float*)D->mom[p ^ 1u]), dev_global(la.flags),
+                       la.nx, la.ny, la.nz, la.plane, la.omega, D->tiles_x, D->tiles_y, D->chunks, m.y);
+}
+
+void launch_sep(Batch& b) {
+  if (b.n_sep <= 0) return;
+  const int2* map = b.d_map + b.n_bc + b.n_wave + b.n_bulk;
+  if (b.options & FF_OPT_PERIODIC) kb_sep3d<true><<<b.n_sep, kSepThreads, 0, b.stream>>>(b.d_doms, map);
+  else kb_sep3d<false><<<b.n_sep, kSepThreads, 0, b.stream>>>(b.d_doms, map);
+}
+
 // Tiles only (the map's tile range), for timing.
 static void launch_bulk_only(Batch& b, int tile, const int2* map, int nblocks) {
   if (b.storage == FF_STORAGE_F32) launch_stream_batch<float>(b, tile, map, nblocks, 0, 0);
@@ -338,14 +365,12 @@ static void tiles_of(const Batch& b, const Domain& d, int tile, int* tx, int* ty
 }
 
 // Records and block maps for the current members and `tile`; uploads them.
-// Map layout: stream launch [boundary cells][wave][tiles], sums launch,
-// finish launch.
+// Map layout: stream launch [boundary cells][wave][tiles], separable launch,
+// sums launch, finish launch.
 static int build_tables(Batch& b, int tile) {
   const int n = (int)b.mem.size();
   std::vector<DomDev> doms(n);
-  std::vector<int2> bc, wave, bulk, es, fin;
-  const int K = b.dim == 2 ? 8 : 26;
-  const int fb = kSumBlock;
+  std::vector<int2> bc, wave, bulk, sep, es, fin;
   const int nt = stream_threads(b.dim, tile);
   int rc = grow(&b.d_steps, &b.steps_cap, (size_t)std::max(n, 1));
   if (rc) return rc;
@@ -364,9 +389,15 @@ static int build_tables(Batch& b, int tile) {
     r.bflag = b.d_flag;
     int tx, ty, ntl;
     tiles_of(b, d, tile, &tx, &ty, &ntl);
+    r.chunks = sep3d_plan(d);  // the form the domain has on its own, so its results are the same
+    if (r.chunks) {
+      tx = (d.nx + kSepTX - 1) / kSepTX;
+      ty = (d.ny + kSepTY - 1) / kSepTY;
+      ntl = tx * ty * r.chunks;
+    }
     r.tiles_x = tx;
     r.tiles_y = ty;
-    for (int t = 0; t < ntl; t++) bulk.push_back(make_int2(i, t));
+    for (int t = 0; t < ntl; t++) (r.chunks ? sep : bulk).push_back(make_int2(i, t));
     if (bnd) {
       r.la.bc_span = nt;  // whole blocks per pass: many domains fill the chip
       r.nbc = boundary_cell_blocks(d, nt);
@@ -390,24 +421,24 @@ static int build_tables(Batch& b, int tile) {
   // multiple of 8 blocks (the wave range is padded) and block p of the range
   // takes tile (p % 8) * ceil(n / 8) + p / 8 of the concatenated list.
   while ((bc.size() + wave.size()) % kXcds) wave.push_back(make_int2(-1, -1));
-  {
-    const size_t nt = bulk.size(), per = (nt + kXcds - 1) / kXcds;
+  for (auto* tiles : {&bulk, &sep}) {
+    const size_t nt = tiles->size(), per = (nt + kXcds - 1) / kXcds;
     std::vector<int2> order(per * kXcds, make_int2(-1, -1));
     for (size_t p = 0; p < order.size(); p++) {
       const size_t t = (p % kXcds) * per + p / kXcds;
-      if (t < nt) order[p] = bulk[t];
+      if (t < nt) order[p] = (*tiles)[t];
     }
-    bulk.swap(order);
+    tiles->swap(order);
   }
   b.n_bc = (int)bc.size();
   b.n_wave = (int)wave.size();
   b.n_bulk = (int)bulk.size();
+  b.n_sep = (int)sep.size();
   b.n_es = (int)es.size();
   b.n_fin = (int)fin.size();
-  (void)fb;
   std::vector<int2> map;
-  map.reserve(bc.size() + wave.size() + bulk.size() + es.size() + fin.size());
-  for (auto* v : {&bc, &wave, &bulk, &es, &fin}) map.insert(map.end(), v->begin(), v->end());
+  map.reserve(bc.size() + wave.size() + bulk.size() + sep.size() + es.size() + fin.size());
+  for (auto* v : {&bc, &wave, &bulk, &sep, &es, &fin}) map.insert(map.end(), v->begin(), v->end());
   if ((size_t)std::max(n, 1) > b.doms_cap || std::max<size_t>(map.size(), 1) > b.map_cap)
     FF_HIP(hipStreamSynchronize(b.stream));  // the old tables may still be read
   if ((rc = grow(&b.d_doms, &b.doms_cap, (size_t)std::max(n, 1)))) return rc;
@@ -828,6 +859,13 @@ int ff_batch_time_bulk(ff_batch* b, int iters, double* avg_ms) {
   ev.clears[1] = &b->tev1;
   FF_HIP(ev.create(2 * (size_t)iters));
   for (int k = 0; k < iters; k++) {
+    if (b->n_sep > 0) {  // two launches: events around them
+      FF_HIP(hipEventRecord(ev[2 * k], b->stream));
+      launch_bulk_only(*b, tile, map, b->n_bulk);
+      launch_sep(*b);
+      FF_HIP(hipEventRecord(ev[2 * k + 1], b->stream));
+      continue;
+    }
     b->tev0 = ev[2 * k];  // the launch's own start and end (launch_timed)
     b->tev1 = ev[2 * k + 1];
     launch_bulk_only(*b, tile, map, b->n_bulk);

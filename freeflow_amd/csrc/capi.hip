@@ -552,6 +552,11 @@ int ff_set_flags(ff_domain* dd, const uint8_t* flags) {
   Domain& d = *dd;
   FF_HIP(hipSetDevice(d.device));
   std::memcpy(d.h_flags.data(), flags, (size_t)d.n);
+  if (d.dim == 3) {
+    unsigned char wall = 0;  // no early exit: the loop vectorises
+    for (long long c = 0; c < d.n; c++) wall |= (unsigned char)((uint8_t)(flags[c] - 5) <= 6 || flags[c] == 3);
+    d.walls3 = wall;
+  }
   FF_HIP(hipStreamSynchronize(d.stream));
   batch_mark_dirty(d.batch);
   links_moved(d);
@@ -1194,7 +1199,7 @@ int ff_autotune(ff_domain* dd, int* tile) {
       if (!keep) t = v;
     }
   } restore{cur, saved};
-  auto launch = [&]() { return d.dim == 2 ? launch_bulk2d(d, in, out) : launch_bulk3d(d, in, out); };
+  auto launch = [&]() { return d.dim == 2 ? launch_bulk2d(d, in, out) : launch_bulk3d_tiles(d, in, out); };
   // rounds over every candidate (clock and cache drift hit all alike); each
   // candidate keeps its fastest round
   std::vector<double> best(n, 1e30);

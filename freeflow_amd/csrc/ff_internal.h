@@ -106,6 +106,7 @@ struct Domain {
   int cur = 0;
   uint8_t* flags = nullptr;
   std::vector<uint8_t> h_flags;
+  bool walls3 = false;  // some flag is a 3D bounce-back wall (is_wall3: 3, 5 to 11)
   // outlets
   OutletCell* outlets = nullptr;
   int n_outlets = 0;
@@ -207,6 +208,7 @@ LinkArgs link_args(Domain& d, const float* v0, const float* v1, const float* u0,
 // launchers (defined in the .hip units)
 int launch_bulk2d(Domain& d, const void* in, void* out);
 int launch_bulk3d(Domain& d, const void* in, void* out);
+int launch_bulk3d_tiles(Domain& d, const void* in, void* out);
 // boundary step: [detect] -> stream (tiles + boundary cells + next kinematics)
 // -> element sums + outlets + boundary-cell copy-back + next step's detection
 // -> finish (vertex forces, wrench)

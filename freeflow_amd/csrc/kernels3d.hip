@@ -142,7 +142,7 @@ int launch_step_stream3d(Domain& d, const void* in, void* out, const LinkArgs& l
   }
 }
 
-int launch_bulk3d(Domain& d, const void* in, void* out) {
+int launch_bulk3d_tiles(Domain& d, const void* in, void* out) {
   switch (d.storage) {
     case FF_STORAGE_F32: return bulk3d_typed<float>(d, in, out);
     case FF_STORAGE_F16: return bulk3d_typed<__half>(d, in, out);
