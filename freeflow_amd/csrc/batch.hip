@@ -115,52 +115,43 @@ constexpr int kGraphSteps = 8;
 template <typename S, bool STAGE, bool PERIODIC, int TX, int TY, int CPT, bool FAST>
 __global__ void __launch_bounds__(256) kb_step2d(const DomDev* __restrict__ doms, const int2* __restrict__ map,
                                                  int n_bc, int n_wave) {
+  __shared__ StepLds<2, 256, Tile2Lds<STAGE, TX, TY, CPT>> lds;
   const int2 m = map[blockIdx.x];
   if (m.x < 0) return;  // padding of the XCD-aware tile order
   const DomDev* D = doms + m.x;
   const unsigned p = *D->step & 1u;
   const int b = blockIdx.x;
   if (b < n_bc) {
-    bcells_body<2, S, STAGE, PERIODIC, 256, FAST>((const S*)D->mom[p], D->la, m.y, D->nbc);
+    bcells_body<2, S, STAGE, PERIODIC, 256, FAST>((const S*)D->mom[p], D->la, m.y, D->nbc, lds.cells);
   } else if (b < n_bc + n_wave) {
     wave_block_body<2, 256, FAST>(D->la, D->fa, m.y);
   } else {
     bulk2d_tile<S, STAGE, PERIODIC, TX, TY, CPT, FAST>(dev_global((const S*)D->mom[p]), dev_global((S*)D->mom[p ^ 1u]),
                                                        dev_global(D->la.flags), D->la.nx, D->la.ny, D->la.plane,
-                                                       D->la.omega, m.y % D->tiles_x, m.y / D->tiles_x);
+                                                       D->la.omega, m.y % D->tiles_x, m.y / D->tiles_x, lds.tile);
   }
 }
 
-// RING = 0: TX x TY x ZC box tiles; otherwise TX x TY columns marching ZC planes; NT = block size.
+// Tile shapes as in tile3d; NT = block size.
 template <typename S, bool PERIODIC, bool FAST, int KIND, int TX, int TY, int ZC, int NT, int PF, bool DMA>
-__global__ void __launch_bounds__(NT) kb_step3d(const DomDev* __restrict__ doms, const int2* __restrict__ map,
-                                                int n_bc, int n_wave) {
+__global__ void __launch_bounds__(NT, (KIND == 2 && !DMA ? 4 : 2))
+    kb_step3d(const DomDev* __restrict__ doms, const int2* __restrict__ map, int n_bc, int n_wave) {
   static_assert(KIND != 2 || NT == ColTile<TX, TY>::NT, "block size of a staged column");
+  __shared__ StepLds<3, NT, Tile3Lds<S, KIND, TX, TY, ZC, PF, DMA>> lds;
   const int2 m = map[blockIdx.x];
   if (m.x < 0) return;  // padding of the XCD-aware tile order
   const DomDev* D = doms + m.x;
   const unsigned p = *D->step & 1u;
   const int b = blockIdx.x;
   if (b < n_bc) {
-    bcells_body<3, S, false, PERIODIC, NT, FAST>((const S*)D->mom[p], D->la, m.y, D->nbc);
+    bcells_body<3, S, false, PERIODIC, NT, FAST>((const S*)D->mom[p], D->la, m.y, D->nbc, lds.cells);
   } else if (b < n_bc + n_wave) {
     wave_block_body<3, NT, FAST>(D->la, D->fa, m.y);
   } else {
-    const int tx = D->tiles_x, ty = D->tiles_y;
-    const int bx = m.y % tx, by = (m.y / tx) % ty, bz = m.y / (tx * ty);
-    const S* in = dev_global((const S*)D->mom[p]);
-    S* out = dev_global((S*)D->mom[p ^ 1u]);
     const LinkArgs& la = D->la;
-    const uint8_t* flags = dev_global(la.flags);
-    if constexpr (KIND == 2)
-      bulk3d_col<S, PERIODIC, FAST, TX, TY, PF, DMA>(in, out, flags, la.nx, la.ny, la.nz, la.plane, la.omega, bx,
-                                                     by, bz * ZC, min(bz * ZC + ZC, la.nz));
-    else if constexpr (KIND == 1)
-      bulk3d_ring<S, PERIODIC, TX, TY, ZC, FAST>(in, out, flags, la.nx, la.ny, la.nz, la.plane, la.omega, bx, by,
-                                                 bz);
-    else
-      bulk3d_tile<S, PERIODIC, TX, TY, ZC, FAST>(in, out, flags, la.nx, la.ny, la.nz, la.plane, la.omega, bx, by,
-                                                 bz);
+    tile3d<S, PERIODIC, FAST, KIND, TX, TY, ZC, PF, DMA>(dev_global((const S*)D->mom[p]), dev_global((S*)D->mom[p ^ 1u]),
+                                                         dev_global(la.flags), la.nx, la.ny, la.nz, la.plane, la.omega,
+                                                         m.y, D->tiles_x, D->tiles_y, lds.tile);
   }
 }
 
@@ -176,13 +167,14 @@ __global__ void __launch_bounds__(FB) kb_sums(const DomDev* __restrict__ doms, c
 template <int DIM, int FB>
 __global__ void __launch_bounds__(FB) kb_finish(const DomDev* __restrict__ doms, const int2* __restrict__ map) {
   const int2 m = map[blockIdx.x];
+  __shared__ FinishLds<DIM> lds;
   const DomDev* D = doms + m.x;
   if (m.y < D->nvb) {
     finish_vertex_body<DIM, FB>(D->la, D->fa, m.y);
     return;
   }
   if (D->boundary) {
-    finish_last_body<DIM, FB>(D->la, D->fa, D->la.st->gen, true);
+    finish_last_body<DIM, FB>(D->la, D->fa, D->la.st->gen, true, lds);
     if (threadIdx.x == 0 && D->la.st->overflow) *D->bflag = 1;
   }
   if (threadIdx.x == 0) *D->step = *D->step + 1u;

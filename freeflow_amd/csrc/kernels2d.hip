@@ -24,9 +24,11 @@ template <typename S, bool STAGE, bool PERIODIC, int TX, int TY, int CPT, bool F
 __global__ void __launch_bounds__(256)
     k_bulk2d(const S* __restrict__ in, S* __restrict__ out, const uint8_t* __restrict__ flags, int nx, int ny,
              size_t plane, float omega, int tiles_x, int ntiles) {
+  __shared__ Tile2Lds<STAGE, TX, TY, CPT> lds;
   const int t = xcd_tile(blockIdx.x, ntiles);
   if (t < 0) return;
-  bulk2d_tile<S, STAGE, PERIODIC, TX, TY, CPT, FAST>(in, out, flags, nx, ny, plane, omega, t % tiles_x, t / tiles_x);
+  bulk2d_tile<S, STAGE, PERIODIC, TX, TY, CPT, FAST>(in, out, flags, nx, ny, plane, omega, t % tiles_x, t / tiles_x,
+                                                     lds);
 }
 
 // Stream launch of a step with a boundary: the first `nbc` blocks update the
@@ -39,16 +41,17 @@ template <typename S, bool STAGE, bool PERIODIC, int TX, int TY, int CPT, bool F
 __global__ void __launch_bounds__(256)
     k_step2d(const S* __restrict__ in, S* __restrict__ out, int tiles_x, int ntiles, int nbc, int nwave, LinkArgs la,
              FinalArgs fa) {
+  __shared__ StepLds<2, 256, Tile2Lds<STAGE, TX, TY, CPT>> lds;
   const int b = blockIdx.x;
   if (b < nbc) {
-    bcells_body<2, S, STAGE, PERIODIC, 256, FAST>(in, la, b, nbc);
+    bcells_body<2, S, STAGE, PERIODIC, 256, FAST>(in, la, b, nbc, lds.cells);
   } else if (b < nbc + nwave) {
-    stream_extra_body<2, 256, FAST>(la, fa, b - nbc);
+    stream_extra_body<2, 256, FAST>(la, fa, b - nbc, lds.finish);
   } else {
     const int t = xcd_tile(b - nbc - nwave, ntiles);
     if (t < 0) return;
     bulk2d_tile<S, STAGE, PERIODIC, TX, TY, CPT, FAST>(in, out, la.flags, la.nx, la.ny, la.plane, la.omega,
-                                                       t % tiles_x, t / tiles_x);
+                                                       t % tiles_x, t / tiles_x, lds.tile);
   }
 }
 

@@ -15,23 +15,6 @@
 
 namespace ff {
 
-// One tile per block (XCD-aware order).  KIND 0: boxes of TX x TY x ZC cells;
-// 1: TX x TY columns marching ZC planes (bulk3d_ring); 2: TX x TY columns
-// marching ZC planes with one staged cell per thread (bulk3d_col: FAST picks
-// its arithmetic, PF and DMA how the next planes' moments are fetched).
-template <typename S, bool PERIODIC, bool FAST, int KIND, int TX, int TY, int ZC, int PF, bool DMA>
-__device__ __forceinline__ void tile3d(const S* in, S* out, const uint8_t* flags, int nx, int ny, int nz, size_t plane,
-                                       float omega, int t, int tiles_x, int tiles_y) {
-  const int bx = t % tiles_x, by = (t / tiles_x) % tiles_y, bz = t / (tiles_x * tiles_y);
-  if constexpr (KIND == 2)
-    bulk3d_col<S, PERIODIC, FAST, TX, TY, PF, DMA>(in, out, flags, nx, ny, nz, plane, omega, bx, by, bz * ZC,
-                                                   min(bz * ZC + ZC, nz));
-  else if constexpr (KIND == 1)
-    bulk3d_ring<S, PERIODIC, TX, TY, ZC, FAST>(in, out, flags, nx, ny, nz, plane, omega, bx, by, bz);
-  else
-    bulk3d_tile<S, PERIODIC, TX, TY, ZC, FAST>(in, out, flags, nx, ny, nz, plane, omega, bx, by, bz);
-}
-
 // Staged columns are built for four waves per SIMD (at most 128 VGPRs); with
 // an LDS ring of moments the LDS allows two or three.
 template <typename S, bool PERIODIC, bool FAST, int KIND, int TX, int TY, int ZC, int NT, int PF, bool DMA>
@@ -39,9 +22,11 @@ __global__ void __launch_bounds__(NT, (KIND == 2 && !DMA ? 4 : 2))
     k_bulk3d(const S* __restrict__ in, S* __restrict__ out, const uint8_t* __restrict__ flags, int nx, int ny,
              int nz, size_t plane, float omega, int tiles_x, int tiles_y, int ntiles) {
   static_assert(KIND != 2 || NT == ColTile<TX, TY>::NT, "block size of a staged column");
+  __shared__ Tile3Lds<S, KIND, TX, TY, ZC, PF, DMA> lds;
   const int t = xcd_tile(blockIdx.x, ntiles);
   if (t < 0) return;
-  tile3d<S, PERIODIC, FAST, KIND, TX, TY, ZC, PF, DMA>(in, out, flags, nx, ny, nz, plane, omega, t, tiles_x, tiles_y);
+  tile3d<S, PERIODIC, FAST, KIND, TX, TY, ZC, PF, DMA>(in, out, flags, nx, ny, nz, plane, omega, t, tiles_x, tiles_y,
+                                                       lds);
 }
 
 template <typename S, bool PERIODIC, bool FAST, int KIND, int TX, int TY, int ZC, int NT, int PF, bool DMA>
@@ -62,20 +47,21 @@ static void bulk3d_variant(Domain& d, const S* i, S* o) {
 // Stream launch of a 3D step with a boundary (see k_step2d): boundary-cell
 // blocks, wave blocks, then the tiles of the chosen shape; NT = block size.
 template <typename S, bool PERIODIC, bool FAST, int KIND, int TX, int TY, int ZC, int NT, int PF, bool DMA>
-__global__ void __launch_bounds__(NT)
+__global__ void __launch_bounds__(NT, (KIND == 2 && !DMA ? 4 : 2))
     k_step3d(const S* __restrict__ in, S* __restrict__ out, int tiles_x, int tiles_y, int ntiles, int nbc, int nwave,
              LinkArgs la, FinalArgs fa) {
   static_assert(KIND != 2 || NT == ColTile<TX, TY>::NT, "block size of a staged column");
+  __shared__ StepLds<3, NT, Tile3Lds<S, KIND, TX, TY, ZC, PF, DMA>> lds;
   const int b = blockIdx.x;
   if (b < nbc) {
-    bcells_body<3, S, false, PERIODIC, NT, FAST>(in, la, b, nbc);
+    bcells_body<3, S, false, PERIODIC, NT, FAST>(in, la, b, nbc, lds.cells);
   } else if (b < nbc + nwave) {
-    stream_extra_body<3, NT, FAST>(la, fa, b - nbc);
+    stream_extra_body<3, NT, FAST>(la, fa, b - nbc, lds.finish);
   } else {
     const int t = xcd_tile(b - nbc - nwave, ntiles);
     if (t < 0) return;
     tile3d<S, PERIODIC, FAST, KIND, TX, TY, ZC, PF, DMA>(in, out, la.flags, la.nx, la.ny, la.nz, la.plane, la.omega,
-                                                         t, tiles_x, tiles_y);
+                                                         t, tiles_x, tiles_y, lds.tile);
   }
 }
 

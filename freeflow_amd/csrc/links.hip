@@ -74,9 +74,10 @@ __global__ void __launch_bounds__(FB) k_step_sums(LinkArgs la, FinalArgs fa, voi
 // i.e. L2 write-back and invalidation, which costs more than the launch.)
 template <int DIM, int FB>
 __global__ void __launch_bounds__(FB) k_step_finish(LinkArgs la, FinalArgs fa, int nvb) {
+  __shared__ FinishLds<DIM> lds;
   const int b = blockIdx.x;
   if (b < nvb) finish_vertex_body<DIM, FB>(la, fa, b);
-  else finish_last_body<DIM, FB>(la, fa, fa.fin_gen, false);
+  else finish_last_body<DIM, FB>(la, fa, fa.fin_gen, false, lds);
 }
 
 // Detection blocks of 256 threads (detect_block).
@@ -96,12 +97,14 @@ int copyback_blocks(const Domain& d, int fb, int per_thread) {
 }
 
 // A domain stepped on its own spreads its boundary cells over about 256
-// blocks (one per CU, few cells each: the launch's latency is the slowest
-// block's), scanning 64..(smallest block size) slots per pass.
+// blocks in 2D and 512 in 3D, where a block takes half as many cells at a
+// time (few cells each: the launch's latency is the slowest block's),
+// scanning 64..(smallest block size) slots per pass.  Smaller spans only add
+// blocks: 16 slots make the 64^3 sphere's 3D launch 21.9 us against 20.8.
 int bc_span(const Domain& d) {
-  const int nt_min = d.dim == 2 ? 256 : 128;
+  const int nt_min = d.dim == 2 ? 256 : 128, blocks = d.dim == 2 ? 256 : 512;
   int s = 64;
-  while (s < nt_min && (long long)s * 256 < d.lt_cap) s *= 2;
+  while (s < nt_min && (long long)s * blocks < d.lt_cap) s *= 2;
   return s;
 }
 

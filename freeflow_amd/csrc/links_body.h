@@ -44,6 +44,13 @@ __device__ __forceinline__ float cell_pop(const float* m, int i) {
   }
 }
 
+template <int DIM, int NT>
+struct CellsLds {
+  static constexpr int CPB = NT / (DIM == 2 ? 16 : 32);
+  float sp[CPB][DIM == 2 ? 9 : 27];
+  int s_slot[NT], s_cell[NT], s_wn[NT / 64], s_upd[CPB];
+};
+
 // The result is written to the cell's side-buffer row (la.sb), not to the
 // output moments: the stream-collide tiles of the same launch also write the
 // cell, and the element-sum launch copies the side buffer over them.
@@ -51,15 +58,19 @@ __device__ __forceinline__ float cell_pop(const float* m, int i) {
 // stride nblk * bc_span), compacts the occupied ones in LDS and updates those
 // cells CPB at a time.
 template <int DIM, typename S, bool STAGE, bool PERIODIC, int NT, bool FAST = false>
-__device__ __forceinline__ void bcells_body(const S* __restrict__ in, const LinkArgs& la, int blk, int nblk) {
+__device__ __forceinline__ void bcells_body(const S* __restrict__ in, const LinkArgs& la, int blk, int nblk,
+                                            CellsLds<DIM, NT>& lds) {
   constexpr int Q = DIM == 2 ? 9 : 27;
   constexpr int K = Q - 1;
   constexpr int NM = DIM == 2 ? 6 : 10;
   constexpr int LPC = DIM == 2 ? 16 : 32;  // lanes per cell
   constexpr int CPB = NT / LPC;            // cells per block
   constexpr int NW = NT / 64;
-  __shared__ float sp[CPB][Q];
-  __shared__ int s_slot[NT], s_cell[NT], s_wn[NW], s_upd[CPB];
+  auto& sp = lds.sp;
+  auto& s_slot = lds.s_slot;
+  auto& s_cell = lds.s_cell;
+  auto& s_wn = lds.s_wn;
+  auto& s_upd = lds.s_upd;
   const unsigned gen = step_gen(la);
   const unsigned tag = step_tag(la);
   const float* v = la.v[gen & 1];
@@ -670,8 +681,15 @@ __device__ __forceinline__ void finish_vertex_body(const LinkArgs& la, const Fin
   }
 }
 
+// LDS of finish_last_body: the wrench's channels and the power of each lane.
+template <int DIM>
+struct FinishLds {
+  double s_red[DIM + (DIM == 2 ? 1 : 3) + 1][kSumLanes];
+};
+
 template <int DIM, int FB>
-__device__ __forceinline__ void finish_last_body(const LinkArgs& la, const FinalArgs& fa, unsigned gen, bool advance) {
+__device__ __forceinline__ void finish_last_body(const LinkArgs& la, const FinalArgs& fa, unsigned gen, bool advance,
+                                                 FinishLds<DIM>& lds) {
   constexpr int NT = DIM == 2 ? 1 : 3;
   constexpr int STRIDE = elem_stride_v<DIM>;
   constexpr int NW = DIM + NT;
@@ -680,7 +698,7 @@ __device__ __forceinline__ void finish_last_body(const LinkArgs& la, const Final
   // body's wrench is the same FP64 number from every launch shape.  Channels:
   // the wrench (NW), then the power.
   constexpr int V = kSumLanes, NC = NW + 1;
-  __shared__ double s_red[NC][V];
+  auto& s_red = lds.s_red;
   for (int bd = 0; bd < fa.n_bodies; bd++) {
     for (int v = threadIdx.x; v < V; v += FB) {
       double a[NC];
@@ -725,14 +743,26 @@ __device__ __forceinline__ void finish_last_body(const LinkArgs& la, const Final
 // The previous step's element sums are complete (earlier launch) and this
 // step's are not started (later launch).
 template <int DIM, int NT, bool FAST = false>
-__device__ __forceinline__ void stream_extra_body(const LinkArgs& la, const FinalArgs& fa, int blk) {
+__device__ __forceinline__ void stream_extra_body(const LinkArgs& la, const FinalArgs& fa, int blk,
+                                                  FinishLds<DIM>& lds) {
   if (blk < fa.kin_blocks) {
     wave_block_body<DIM, NT, FAST>(la, fa, blk);
     return;
   }
   blk -= fa.kin_blocks;
   if (blk < fa.fin_blocks - 1) finish_vertex_body<DIM, NT>(la, fa, blk);
-  else finish_last_body<DIM, NT>(la, fa, fa.fin_gen, false);
+  else finish_last_body<DIM, NT>(la, fa, fa.fin_gen, false, lds);
 }
+
+// LDS of a stream launch: its blocks are tiles, boundary-cell blocks or
+// extras, and share it.  (Each with its own, a 3D launch had 17 KB more and
+// held one box or two 16x12x8 columns a CU instead of two or four: 160x96x96
+// around a sphere 125 us against 74 with boxes, 55 against 45 with columns.)
+template <int DIM, int NT, class TILE>
+union StepLds {
+  TILE tile;
+  CellsLds<DIM, NT> cells;
+  FinishLds<DIM> finish;
+};
 
 }  // namespace ff

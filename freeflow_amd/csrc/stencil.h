@@ -36,6 +36,14 @@ struct Tile2 {
 constexpr Tile2 kTiles2[] = {{32, 8, 1}, {32, 8, 2}, {64, 4, 2}, {32, 8, 4}, {64, 4, 4}};
 constexpr int kNumTiles2 = 5;
 
+// LDS of the tile bodies below: the caller's, so that launches with other
+// kinds of blocks share it with theirs (a kernel's LDS is what its blocks
+// need at most, not the sum over their kinds).
+template <bool STAGE, int TX, int TY, int CPT>
+struct Tile2Lds {
+  typename std::conditional<STAGE, __half, float>::type sp[9][(TX + 2) * (TY * CPT + 2)];
+};
+
 // Stage the reconstructed populations of the tile and its one-cell halo in
 // LDS (clamped or periodic halo; binary16 when the reference's half tile is
 // reproduced), then pull, collide and store every updated cell.  FAST picks
@@ -43,12 +51,11 @@ constexpr int kNumTiles2 = 5;
 template <typename S, bool STAGE, bool PERIODIC, int TX, int TY, int CPT, bool FAST = false>
 __device__ __forceinline__ void bulk2d_tile(const S* __restrict__ in, S* __restrict__ out,
                                             const uint8_t* __restrict__ flags, int nx, int ny, size_t plane,
-                                            float omega, int bx, int by) {
+                                            float omega, int bx, int by, Tile2Lds<STAGE, TX, TY, CPT>& lds) {
   constexpr int NT = TX * TY, RY = TY * CPT;
   constexpr int HX = TX + 2, HY = RY + 2, HN = HX * HY;
-  using T = typename std::conditional<STAGE, __half, float>::type;
   constexpr int PER = (HN + NT - 1) / NT;  // halo cells per thread
-  __shared__ T sp[9][HN];
+  auto& sp = lds.sp;
   const int x0 = bx * TX, y0 = by * RY;
   // every load of the tile is issued before the first reconstruction, so the
   // block waits for memory once
@@ -113,6 +120,14 @@ __device__ __forceinline__ void bulk2d_tile(const S* __restrict__ in, S* __restr
   }
 }
 
+template <int TX, int TY, int TZ>
+struct Box3Lds {
+  static constexpr int HN = (TX + 2) * (TY + 2) * (TZ + 2);
+  float sp[27][HN];
+  int swall[(TX * TY * TZ + 63) / 64];  // per wave: a staged cell is a bounce-back wall
+  uint8_t sf[HN];
+};
+
 // 3D box tile of TX x TY x TZ cells (one per thread) with a one-cell halo in
 // LDS (FP32 as the reference's tile, FsiCoupling3D.cu:94).  The reference
 // keeps the flag bounce-back value in 3D (FsiCoupling3D.cu:209-222), so
@@ -120,15 +135,15 @@ __device__ __forceinline__ void bulk2d_tile(const S* __restrict__ in, S* __restr
 template <typename S, bool PERIODIC, int TX, int TY, int TZ, bool FAST = false>
 __device__ __forceinline__ void bulk3d_tile(const S* __restrict__ in, S* __restrict__ out,
                                             const uint8_t* __restrict__ flags, int nx, int ny, int nz, size_t plane,
-                                            float omega, int bx, int by, int bz) {
+                                            float omega, int bx, int by, int bz, Box3Lds<TX, TY, TZ>& lds) {
   constexpr int kTX3 = TX, kTY3 = TY, kTZ3 = TZ;
   constexpr int HX = kTX3 + 2, HY = kTY3 + 2, HZ = kTZ3 + 2, HN = HX * HY * HZ;
   constexpr int NT = kTX3 * kTY3 * kTZ3;
   constexpr int PER = (HN + NT - 1) / NT;  // halo cells per thread
   constexpr int NW = (NT + 63) / 64;
-  __shared__ float sp[27][HN];
-  __shared__ uint8_t sf[HN];
-  __shared__ int swall[NW];  // per wave: a staged cell is a bounce-back wall
+  auto& sp = lds.sp;
+  auto& sf = lds.sf;
+  auto& swall = lds.swall;
   const int x0 = bx * kTX3, y0 = by * kTY3, z0 = bz * kTZ3;
   // all loads first, then the reconstructions (one wait for memory)
   float m[PER][10];
@@ -260,19 +275,29 @@ __host__ __device__ constexpr int zclass_index(int i) {
   return n;
 }
 
+// rel = z - z0 + 1 numbers the planes from the lower halo plane
+template <int TX, int TY>
+struct Ring3Lds {
+  static constexpr int HA = (TX + 2) * (TY + 2);
+  float sup[2][9][HA];                // c_z = +1 class, slot rel % 2
+  float szc[9][HA];                   // c_z = 0 class of the current plane
+  float sdn[2][9][HA];                // c_z = -1 class, slot rel % 2
+  int swall[3][(TX * TY + 63) / 64];  // per flag slot and wave: a staged cell is a wall
+  uint8_t sf[3][HA];                  // flags, slot rel % 3
+};
+
 template <typename S, bool PERIODIC, int TX, int TY, int ZC, bool FAST = false>
 __device__ __forceinline__ void bulk3d_ring(const S* __restrict__ in, S* __restrict__ out,
                                             const uint8_t* __restrict__ flags, int nx, int ny, int nz, size_t plane,
-                                            float omega, int bx, int by, int bz) {
+                                            float omega, int bx, int by, int bz, Ring3Lds<TX, TY>& lds) {
   constexpr int NT = TX * TY, HX = TX + 2, HY = TY + 2, HA = HX * HY;
   constexpr int PER = (HA + NT - 1) / NT;  // halo cells per thread per plane
   constexpr int NW = (NT + 63) / 64;
-  // rel = z - z0 + 1 numbers the planes from the lower halo plane
-  __shared__ float sup[2][9][HA];  // c_z = +1 class, slot rel % 2
-  __shared__ float szc[9][HA];     // c_z = 0 class of the current plane
-  __shared__ float sdn[2][9][HA];  // c_z = -1 class, slot rel % 2
-  __shared__ uint8_t sf[3][HA];    // flags, slot rel % 3
-  __shared__ int swall[3][NW];     // per flag slot and wave: a staged cell is a wall
+  auto& sup = lds.sup;
+  auto& szc = lds.szc;
+  auto& sdn = lds.sdn;
+  auto& sf = lds.sf;
+  auto& swall = lds.swall;
   const int x0 = bx * TX, y0 = by * TY, z0 = bz * ZC;
   const int zend = min(z0 + ZC, nz);
   float mreg[PER][10];
@@ -427,6 +452,18 @@ struct ColTile {
   static constexpr int NT = (HA + 63) / 64 * 64;  // block size
 };
 
+template <typename S, int TX, int TY, int PF, bool DMA>
+struct Col3Lds {
+  static constexpr int HA = ColTile<TX, TY>::HA, NT = ColTile<TX, TY>::NT;
+  static constexpr bool USE_DMA = DMA && std::is_same<S, float>::value;
+  float ring[USE_DMA ? PF : 1][USE_DMA ? 10 : 1][USE_DMA ? NT : 1];  // moments of the planes in flight
+  float sup[2][9][HA];    // c_z = +1 class, slot rel & 1
+  float szc[9][HA];       // c_z = 0 class of plane z
+  float sdn[9][HA];       // c_z = -1 class of plane z + 1
+  int swall[3][NT / 64];  // per flag slot and wave: a staged cell is a wall
+  uint8_t sf[3][HA];      // flags, slot rel % 3
+};
+
 // PF planes of moments are in flight while a plane is computed: in registers,
 // or (DMA, FP32 storage) in an LDS ring of PF planes filled by LDS DMA loads
 // (global_load_lds: the load writes LDS without passing through VGPRs, so
@@ -434,19 +471,20 @@ struct ColTile {
 template <typename S, bool PERIODIC, bool FAST, int TX, int TY, int PF = 1, bool DMA = false>
 __device__ __forceinline__ void bulk3d_col(const S* __restrict__ in, S* __restrict__ out,
                                            const uint8_t* __restrict__ flags, int nx, int ny, int nz, size_t plane,
-                                           float omega, int bx, int by, int z0, int zend) {
+                                           float omega, int bx, int by, int z0, int zend,
+                                           Col3Lds<S, TX, TY, PF, DMA>& lds) {
   using CT = ColTile<TX, TY>;
   constexpr int HX = CT::HX, HY = CT::HY, HA = CT::HA, NI = CT::NI, NW = CT::NT / 64;
   constexpr bool USE_DMA = DMA && std::is_same<S, float>::value;
   static_assert(PF >= 1 && PF <= 4, "planes in flight");
   // 16-bit storage loads through registers: one plane in flight for a DMA shape
   constexpr int NP = (DMA && !USE_DMA) ? 1 : PF;
-  __shared__ float ring[USE_DMA ? NP : 1][10][USE_DMA ? CT::NT : 1];  // moments of the planes in flight
-  __shared__ float sup[2][9][HA];  // c_z = +1 class, slot rel & 1
-  __shared__ float szc[9][HA];     // c_z = 0 class of plane z
-  __shared__ float sdn[9][HA];     // c_z = -1 class of plane z + 1
-  __shared__ uint8_t sf[3][HA];    // flags, slot rel % 3
-  __shared__ int swall[3][NW];     // per flag slot and wave: a staged cell is a wall
+  auto& ring = lds.ring;
+  auto& sup = lds.sup;
+  auto& szc = lds.szc;
+  auto& sdn = lds.sdn;
+  auto& sf = lds.sf;
+  auto& swall = lds.swall;
   const int t = threadIdx.x;
   __syncthreads();  // a block may run several columns in turn: the last one's reads are done
   // staged cell (hx, hy) of this thread in the (TX+2) x (TY+2) halo frame
@@ -686,6 +724,30 @@ __device__ __forceinline__ void bulk3d_col(const S* __restrict__ in, S* __restri
       if (z + 3 < zend) plane_step(z + 3, std::integral_constant<int, (NP > 3 ? 3 : 0)>{});
   }
   flush();  // the last plane
+}
+
+// LDS of a 3D tile by its kind (FF_TILES3).
+template <typename S, int KIND, int TX, int TY, int ZC, int PF, bool DMA>
+using Tile3Lds = typename std::conditional<
+    KIND == 2, Col3Lds<S, TX, TY, PF, DMA>,
+    typename std::conditional<KIND == 1, Ring3Lds<TX, TY>, Box3Lds<TX, TY, ZC>>::type>::type;
+
+// Tile t of a grid of tiles_x x tiles_y x ... tiles.  KIND 0: boxes of TX x TY x ZC cells;
+// 1: TX x TY columns marching ZC planes (bulk3d_ring); 2: TX x TY columns
+// marching ZC planes with one staged cell per thread (bulk3d_col: FAST picks
+// its arithmetic, PF and DMA how the next planes' moments are fetched).
+template <typename S, bool PERIODIC, bool FAST, int KIND, int TX, int TY, int ZC, int PF, bool DMA>
+__device__ __forceinline__ void tile3d(const S* in, S* out, const uint8_t* flags, int nx, int ny, int nz, size_t plane,
+                                       float omega, int t, int tiles_x, int tiles_y,
+                                       Tile3Lds<S, KIND, TX, TY, ZC, PF, DMA>& lds) {
+  const int bx = t % tiles_x, by = (t / tiles_x) % tiles_y, bz = t / (tiles_x * tiles_y);
+  if constexpr (KIND == 2)
+    bulk3d_col<S, PERIODIC, FAST, TX, TY, PF, DMA>(in, out, flags, nx, ny, nz, plane, omega, bx, by, bz * ZC,
+                                                   min(bz * ZC + ZC, nz), lds);
+  else if constexpr (KIND == 1)
+    bulk3d_ring<S, PERIODIC, TX, TY, ZC, FAST>(in, out, flags, nx, ny, nz, plane, omega, bx, by, bz, lds);
+  else
+    bulk3d_tile<S, PERIODIC, TX, TY, ZC, FAST>(in, out, flags, nx, ny, nz, plane, omega, bx, by, bz, lds);
 }
 
 }  // namespace ff
