@@ -1220,7 +1220,7 @@ int ff_autotune(ff_domain* dd, int* tile) {
   const int best_t = (int)(std::min_element(best.begin(), best.end()) - best.begin());
   cur = rc ? saved : best_t;
   restore.keep = true;
-  if (tile) *tile = cur;
+  if (tile) *tile = std::max(cur, 0);
   return rc;
 }
 
