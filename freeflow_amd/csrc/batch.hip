@@ -73,7 +73,7 @@ struct Batch {
   unsigned* d_steps = nullptr;
   size_t steps_cap = 0;
   int n_bc = 0, n_wave = 0, n_bulk = 0, n_sep = 0, n_es = 0, n_fin = 0;
-  int* d_flag = nullptr;  // set by a replay whose detection overflowed a member's link table
+  int* d_flag = nullptr;  // pinned: set by a replay whose detection overflowed a member's link table
   // pending detections (members whose links were not detected ahead): pinned
   // staging and its device copy, reused or regrown only once the copy and the
   // launches that read it (pend_ev) have completed
@@ -698,14 +698,13 @@ int ff_batch_create(int dim, int storage, unsigned options, int device, ff_batch
     delete b;
     return hip_fail(e, "hipStreamCreate");
   }
-  e = hipMalloc((void**)&b->d_flag, 256);
-  if (e == hipSuccess) e = hipMemset(b->d_flag, 0, 256);
+  e = hipHostMalloc((void**)&b->d_flag, sizeof(int), hipHostMallocDefault);
   if (e != hipSuccess) {
-    if (b->d_flag) (void)hipFree(b->d_flag);
     (void)hipStreamDestroy(b->stream);
     delete b;
     return hip_fail(e, "batch flag");
   }
+  *b->d_flag = 0;
   *out = b;
   return FF_OK;
 }
@@ -719,7 +718,7 @@ int ff_batch_destroy(ff_batch* b) {
   if (b->d_doms) (void)hipFree(b->d_doms);
   if (b->d_map) (void)hipFree(b->d_map);
   if (b->d_steps) (void)hipFree(b->d_steps);
-  if (b->d_flag) (void)hipFree(b->d_flag);
+  (void)hipHostFree(b->d_flag);
   if (b->d_pend) (void)hipFree(b->d_pend);
   if (b->h_pend) (void)hipHostFree(b->h_pend);
   if (b->pend_ev) (void)hipEventDestroy(b->pend_ev);
@@ -787,9 +786,8 @@ int ff_batch_sync(ff_batch* b) {
   FF_CHECK_BATCH(b);
   FF_HIP(hipSetDevice(b->device));
   FF_HIP(hipStreamSynchronize(b->stream));
-  int flag = 0;  // sticky, like a member's own overflow flag
-  FF_HIP(hipMemcpy(&flag, b->d_flag, sizeof(int), hipMemcpyDeviceToHost));
-  if (flag) return fail(FF_ERR_CAPACITY, "boundary link table overflow in a batched domain");
+  if (*(volatile int*)b->d_flag)  // sticky, like a member's own overflow flag
+    return fail(FF_ERR_CAPACITY, "boundary link table overflow in a batched domain");
   return FF_OK;
 }
 

@@ -97,6 +97,39 @@ struct Carve {
   }
 };
 
+// The histories of the wrenches and powers: a pinned piece that the finish
+// kernels write across the link and readings take without a copy (a reading
+// of a batch's 64 members was 128 copies of 15 us), or device memory where
+// they are large or no pinned memory is left.
+static void free_history(Domain& d) {
+  if (d.hist_pinned) pinned_piece_free(d.wrench_hist);
+  else {
+    dfree(d.wrench_hist);
+    dfree(d.power_hist);
+  }
+  d.wrench_hist = d.power_hist = nullptr;
+  d.hist_pinned = false;
+  d.hist_cap = 0;
+  d.hist_count = 0;
+}
+
+// The latest `n` records of `rec` doubles of a history ring, oldest first
+// (the domain's work is done).
+static int read_history(const Domain& d, const double* ring, size_t rec, int n, double* out) {
+  for (int k = 0; k < n;) {
+    // the step with generation g wrote slot (g - 1) % cap; the latest step is gen_host - 1
+    const long long slot = ((long long)d.gen_host - n + k - 1) % d.hist_cap;
+    const int run = (int)std::min<long long>(n - k, d.hist_cap - slot);
+    double* to = out + (size_t)k * rec;
+    const double* from = ring + (size_t)slot * rec;
+    const size_t bytes = (size_t)run * rec * sizeof(double);
+    if (d.hist_pinned) std::memcpy(to, from, bytes);
+    else FF_HIP(hipMemcpy(to, from, bytes, hipMemcpyDeviceToHost));
+    k += run;
+  }
+  return FF_OK;
+}
+
 static void free_boundary(Domain& d) {
   // the arrays set up by ff_set_boundary share one allocation
   dfree(d.bnd_mem);
@@ -107,8 +140,7 @@ static void free_boundary(Domain& d) {
   d.lt_cells = d.lt_keys = nullptr; d.lk_f = d.lk_b = d.lk_h = d.lk_sb = nullptr;
   d.st = nullptr; d.vert_body = nullptr;
   d.rest_verts = nullptr; d.s_coord = nullptr; d.wave_params = nullptr;
-  dfree(d.wrench_hist);
-  dfree(d.power_hist);
+  free_history(d);
   d.power = nullptr;
   d.nv = d.ne = d.n_bodies = 0;
   d.gen_host = 1;
@@ -116,8 +148,6 @@ static void free_boundary(Domain& d) {
   d.finish_pending = false;
   d.has_boundary = false;
   d.wave = false;
-  d.hist_cap = 0;
-  d.hist_count = 0;
   d.predetected = false;
   d.stale = false;
 }
@@ -429,10 +459,11 @@ static int one_step(Domain& d, const float* pv, const float* pu, const uint32_t*
   return FF_OK;
 }
 
-static int check_overflow(Domain& d) {
-  if (!d.has_boundary) return FF_OK;
-  StepState st;
-  FF_HIP(hipMemcpy(&st, d.st, sizeof(st), hipMemcpyDeviceToHost));
+// Reads the spans together with the overflow flag of the link table.
+static int read_checked(Domain& d, const void* dev = nullptr, void* host = nullptr, size_t bytes = 0) {
+  StepState st{};
+  const Span spans[2] = {{dev, host, bytes}, {d.st, &st, d.has_boundary ? sizeof(st) : 0}};
+  if (int rc = read_spans(d, spans, 2)) return rc;
   if (st.overflow) {
     int z = 0;
     FF_HIP(hipMemcpy(&d.st->overflow, &z, sizeof(int), hipMemcpyHostToDevice));
@@ -510,6 +541,7 @@ int ff_domain_create(const ff_domain_desc* desc, ff_domain** out) {
   d.h_flags.assign((size_t)n, kFluid);
   hipError_t e = acquire_stream(d.device, &d.stream);
   if (e != hipSuccess) { delete dd; return hip_fail(e, "hipStreamCreate"); }
+  pinned_retain();
   // one allocation: both moment buffers (cleared), the flags (Fluid) and the
   // reduction scratch
   Carve cv;
@@ -542,6 +574,7 @@ int ff_domain_destroy(ff_domain* dd) {
   d.red = nullptr;
   dfree(d.outlets);
   release_stream(d.device, d.stream);
+  pinned_release();
   delete dd;
   return FF_OK;
 }
@@ -614,19 +647,8 @@ int ff_get_moments(ff_domain* dd, float* aos, int which) {
   if (which < 0 || which > 1) return fail(FF_ERR_INVALID, "which must be 0 or 1");
   Domain& d = *dd;
   FF_HIP(hipSetDevice(d.device));
-  float* tmp = nullptr;
-  const size_t cnt = (size_t)d.n * d.nm;
-  int rc = dalloc(&tmp, cnt);
-  if (rc) return rc;
-  rc = launch_convert_out(d, d.mom[which == 0 ? d.cur : (d.cur ^ 1)], tmp);
-  if (!rc) {
-    hipError_t e = hipStreamSynchronize(d.stream);
-    if (e == hipSuccess) e = hipMemcpy(aos, tmp, cnt * sizeof(float), hipMemcpyDeviceToHost);
-    if (e != hipSuccess) rc = hip_fail(e, "download moments");
-  }
-  dfree(tmp);
-  if (!rc) rc = check_overflow(d);
-  return rc;
+  if (int rc = read_moments(d, d.mom[which == 0 ? d.cur : (d.cur ^ 1)], aos)) return rc;
+  return d.has_boundary ? read_checked(d) : FF_OK;
 }
 
 int ff_set_boundary(ff_domain* dd, int nv, const float* verts, const float* vels, int ne, const uint32_t* elems,
@@ -827,14 +849,13 @@ int ff_get_vertex_forces(ff_domain* dd, float* out, int reset) {
   if (!out) return fail(FF_ERR_INVALID, "null output");
   FF_HIP(hipSetDevice(d.device));
   if (int frc = flush_finish(d)) return frc;  // the last step's deferred finish
-  FF_HIP(hipStreamSynchronize(d.stream));
   const size_t bytes = (size_t)d.nv * d.dim * sizeof(float);
-  FF_HIP(hipMemcpy(out, d.vforce, bytes, hipMemcpyDeviceToHost));
-  if (reset) {
+  const int rc = read_checked(d, d.vforce, out, bytes);
+  if (reset && (!rc || rc == FF_ERR_CAPACITY)) {
     FF_HIP(hipMemsetAsync(d.vforce, 0, bytes, d.stream));
     FF_HIP(hipStreamSynchronize(d.stream));
   }
-  return check_overflow(d);
+  return rc;
 }
 
 int ff_get_step_vertex_forces(ff_domain* dd, float* out) {
@@ -848,17 +869,8 @@ int ff_get_step_vertex_forces(ff_domain* dd, float* out) {
     std::memset(out, 0, cnt * sizeof(float));
     return FF_OK;
   }
-  float* tmp = nullptr;
-  int rc = dalloc(&tmp, cnt);
-  if (rc) return rc;
-  rc = launch_step_vertex_forces(d, tmp);
-  if (!rc) {
-    hipError_t e = hipStreamSynchronize(d.stream);
-    if (e == hipSuccess) e = hipMemcpy(out, tmp, cnt * sizeof(float), hipMemcpyDeviceToHost);
-    if (e != hipSuccess) rc = hip_fail(e, "step vertex forces");
-  }
-  dfree(tmp);
-  return rc;
+  return read_kernel_output(d, cnt * sizeof(float), out,
+                            [](Domain& dm, void* to) { return launch_step_vertex_forces(dm, (float*)to); });
 }
 
 // ---------------------------------------------------------------- no-allocation readback
@@ -919,9 +931,7 @@ int ff_get_body_wrench(ff_domain* dd, double* out) {
   if (!out) return fail(FF_ERR_INVALID, "null output");
   FF_HIP(hipSetDevice(d.device));
   if (int frc = flush_finish(d)) return frc;  // the last step's deferred finish
-  FF_HIP(hipStreamSynchronize(d.stream));
-  FF_HIP(hipMemcpy(out, d.wrench, (size_t)d.n_bodies * wrench_width(d.dim) * sizeof(double), hipMemcpyDeviceToHost));
-  return check_overflow(d);
+  return read_checked(d, d.wrench, out, (size_t)d.n_bodies * wrench_width(d.dim) * sizeof(double));
 }
 
 int ff_set_wrench_history(ff_domain* dd, int capacity) {
@@ -933,13 +943,17 @@ int ff_set_wrench_history(ff_domain* dd, int capacity) {
   if (int frc = flush_finish(d)) return frc;  // the last step's deferred finish
   FF_HIP(hipStreamSynchronize(d.stream));
   batch_mark_dirty(d.batch);
-  dfree(d.wrench_hist);
-  dfree(d.power_hist);
-  d.hist_cap = 0;
-  d.hist_count = 0;
+  free_history(d);
   if (capacity == 0) return FF_OK;
-  int rc = dalloc(&d.wrench_hist, (size_t)capacity * d.n_bodies * wrench_width(d.dim));
-  if (!rc) rc = dalloc(&d.power_hist, (size_t)capacity * d.n_bodies);
+  const size_t nw = (size_t)capacity * d.n_bodies * wrench_width(d.dim), np = (size_t)capacity * d.n_bodies;
+  if ((d.wrench_hist = (double*)pinned_piece((nw + np) * sizeof(double)))) {
+    d.power_hist = d.wrench_hist + nw;
+    d.hist_pinned = true;
+    d.hist_cap = capacity;
+    return FF_OK;
+  }
+  int rc = dalloc(&d.wrench_hist, nw);
+  if (!rc) rc = dalloc(&d.power_hist, np);
   if (rc) {
     dfree(d.wrench_hist);
     dfree(d.power_hist);
@@ -958,14 +972,7 @@ int ff_get_wrench_history(ff_domain* dd, double* out, int count, int* n_out) {
   FF_HIP(hipStreamSynchronize(d.stream));
   const long long avail = std::min<long long>(d.hist_count, d.hist_cap);
   const int n = (int)std::min<long long>(avail, count);
-  const size_t rec = (size_t)d.n_bodies * wrench_width(d.dim);
-  std::vector<double> ring((size_t)d.hist_cap * rec);
-  if (d.hist_cap) FF_HIP(hipMemcpy(ring.data(), d.wrench_hist, ring.size() * sizeof(double), hipMemcpyDeviceToHost));
-  for (int k = 0; k < n; k++) {
-    // the step with generation g wrote slot (g - 1) % cap; the latest step is gen_host - 1
-    const long long g = (long long)d.gen_host - n + k;
-    std::memcpy(out + (size_t)k * rec, ring.data() + (size_t)((g - 1) % d.hist_cap) * rec, rec * sizeof(double));
-  }
+  if (int rc = read_history(d, d.wrench_hist, (size_t)d.n_bodies * wrench_width(d.dim), n, out)) return rc;
   *n_out = n;
   return FF_OK;
 }
@@ -977,9 +984,7 @@ int ff_get_body_power(ff_domain* dd, double* out) {
   if (!out) return fail(FF_ERR_INVALID, "null output");
   FF_HIP(hipSetDevice(d.device));
   if (int frc = flush_finish(d)) return frc;  // the last step's deferred finish
-  FF_HIP(hipStreamSynchronize(d.stream));
-  FF_HIP(hipMemcpy(out, d.power, (size_t)d.n_bodies * sizeof(double), hipMemcpyDeviceToHost));
-  return check_overflow(d);
+  return read_checked(d, d.power, out, (size_t)d.n_bodies * sizeof(double));
 }
 
 int ff_get_power_history(ff_domain* dd, double* out, int count, int* n_out) {
@@ -991,14 +996,7 @@ int ff_get_power_history(ff_domain* dd, double* out, int count, int* n_out) {
   FF_HIP(hipStreamSynchronize(d.stream));
   const long long avail = std::min<long long>(d.hist_count, d.hist_cap);
   const int n = (int)std::min<long long>(avail, count);
-  const size_t rec = (size_t)d.n_bodies;
-  std::vector<double> ring((size_t)d.hist_cap * rec);
-  if (d.hist_cap) FF_HIP(hipMemcpy(ring.data(), d.power_hist, ring.size() * sizeof(double), hipMemcpyDeviceToHost));
-  for (int k = 0; k < n; k++) {
-    // the step with generation g wrote slot (g - 1) % cap; the latest step is gen_host - 1
-    const long long g = (long long)d.gen_host - n + k;
-    std::memcpy(out + (size_t)k * rec, ring.data() + (size_t)((g - 1) % d.hist_cap) * rec, rec * sizeof(double));
-  }
+  if (int rc = read_history(d, d.power_hist, (size_t)d.n_bodies, n, out)) return rc;
   *n_out = n;
   return FF_OK;
 }
@@ -1008,13 +1006,11 @@ int ff_get_boundary(ff_domain* dd, float* verts, float* vels) {
   Domain& d = *dd;
   if (!d.has_boundary) return fail(FF_ERR_STATE, "no boundary set");
   FF_HIP(hipSetDevice(d.device));
-  FF_HIP(hipStreamSynchronize(d.stream));
   const size_t bytes = (size_t)d.nv * d.dim * sizeof(float);
   // the buffer of the most recent step (both buffers agree before the first)
   const int b = d.gen_host > 1 ? (int)((d.gen_host - 1) & 1) : (int)(d.gen_host & 1);
-  if (verts) FF_HIP(hipMemcpy(verts, d.vbuf[b], bytes, hipMemcpyDeviceToHost));
-  if (vels) FF_HIP(hipMemcpy(vels, d.ubuf[b], bytes, hipMemcpyDeviceToHost));
-  return FF_OK;
+  const Span spans[2] = {{d.vbuf[b], verts, verts ? bytes : 0}, {d.ubuf[b], vels, vels ? bytes : 0}};
+  return read_spans(d, spans, 2);
 }
 
 int ff_mass(ff_domain* dd, double* out) {
@@ -1022,17 +1018,7 @@ int ff_mass(ff_domain* dd, double* out) {
   if (!out) return fail(FF_ERR_INVALID, "null output");
   Domain& d = *dd;
   FF_HIP(hipSetDevice(d.device));
-  double* dev = nullptr;
-  int rc = dalloc(&dev, 1);
-  if (rc) return rc;
-  rc = launch_mass(d, dev);
-  if (!rc) {
-    hipError_t e = hipStreamSynchronize(d.stream);
-    if (e == hipSuccess) e = hipMemcpy(out, dev, sizeof(double), hipMemcpyDeviceToHost);
-    if (e != hipSuccess) rc = hip_fail(e, "mass");
-  }
-  dfree(dev);
-  return rc;
+  return read_kernel_output(d, sizeof(double), out, [](Domain& dm, void* to) { return launch_mass(dm, (double*)to); });
 }
 
 int ff_fill_solid(ff_domain* dd) {
@@ -1051,8 +1037,9 @@ int ff_fill_solid(ff_domain* dd) {
 int ff_sync(ff_domain* dd) {
   FF_CHECK_DOMAIN(dd);
   FF_HIP(hipSetDevice(dd->device));
+  if (dd->has_boundary) return read_checked(*dd);
   FF_HIP(hipStreamSynchronize(dd->stream));
-  return check_overflow(*dd);
+  return FF_OK;
 }
 
 int ff_time_bulk_kernel(ff_domain* dd, int iters, double* avg_ms) {
@@ -1110,7 +1097,7 @@ int ff_time_steps(ff_domain* dd, int nsteps, double* total_ms) {
   FF_HIP(hipEventElapsedTime(&ms, ev[0], ev[1]));
   *total_ms = ms;
   if (rc) return rc;
-  return check_overflow(d);
+  return read_checked(d);
 }
 
 int ff_step_timed(ff_domain* dd, int nsteps, double* total_ms, double* stream_ms) {
@@ -1146,7 +1133,7 @@ int ff_step_timed(ff_domain* dd, int nsteps, double* total_ms, double* stream_ms
     sum += k;
   }
   *stream_ms = sum;
-  return check_overflow(d);
+  return read_checked(d);
 }
 
 int ff_domain_footprint(const ff_domain_desc* desc, int nv, int ne, const float* verts, const uint32_t* elems,

@@ -126,6 +126,7 @@ struct Domain {
   double* body_ref = nullptr;     // n_bodies * dim
   double* elem_acc = nullptr;     // per element: dim*dim vertex shares, dim force, torque
   double* wrench = nullptr;       // n_bodies * (2D:3, 3D:6), latest step
+  bool hist_pinned = false;      // wrench_hist and power_hist share a pinned piece of host memory
   double* wrench_hist = nullptr;  // ring of hist_cap steps
   double* power = nullptr;        // n_bodies: latest step's sum over the body of -F_v . u_v
   double* power_hist = nullptr;   // ring of hist_cap steps
@@ -241,7 +242,21 @@ int detect_blocks(const Domain& d, bool batched);  // detection blocks of 256 th
 int bc_span(const Domain& d);  // boundary-cell scan span of a domain stepped on its own
 int launch_step_vertex_forces(Domain& d, float* out_dev);
 int launch_convert_in(Domain& d, const float* aos_dev, void* buf);
-int launch_convert_out(Domain& d, const void* buf, float* aos_dev);
+// readback.hip.  Spans (multiples of 4 bytes, at most four) and kernel results
+// arrive once the domain's queued work is done.
+struct Span {
+  const void* dev;
+  void* host;
+  size_t bytes;
+};
+int read_spans(Domain& d, const Span* spans, int n);
+int read_kernel_output(Domain& d, size_t bytes, void* out, int (*launch)(Domain&, void*));
+int read_moments(Domain& d, const void* buf, float* out);
+void pinned_retain();  // one per domain: idle pinned blocks are kept while any lives
+void pinned_release();
+constexpr size_t kPinnedPiece = 64u << 10;
+void* pinned_piece(size_t bytes);  // null: larger than kPinnedPiece, or no pinned memory left
+void pinned_piece_free(void* p);
 int launch_mass(Domain& d, double* out_dev);
 int launch_fill_solid(Domain& d, const float* verts);
 

@@ -128,14 +128,16 @@ void bind_simulator(py::module_& m, const char* name) {
       .def(
           "get_fluid_moments",
           [](const S& s) {
-            const std::vector<float> mom = s.getFluidMoment(0);
+            s.fluidMomentCount();  // throws before initialize()
             const auto& p = s.m_params;
             std::vector<py::ssize_t> shape;
             if constexpr (D == 2)
               shape = {p.fluid_ny, p.fluid_nx, 6};
             else
               shape = {p.fluid_nz, p.fluid_ny, p.fluid_nx, 10};
-            return py::array_t<float>(shape, mom.data());
+            py::array_t<float> mom(shape);
+            s.readFluidMoment(0, mom.mutable_data());
+            return mom;
           },
           "Get the current fluid moment fields.")
       .def("getVertices", [](const S& s) { return rows<D>(s.getVertices()); }, "Get the position of solid vertices")
@@ -173,8 +175,9 @@ void bind_simulator(py::module_& m, const char* name) {
       .def(
           "get_fluid_moments_buffer",
           [](const S& s, int which) {
-            const std::vector<float> mom = s.getFluidMoment(which);
-            return py::array_t<float>((py::ssize_t)mom.size(), mom.data());
+            py::array_t<float> mom((py::ssize_t)s.fluidMomentCount());
+            s.readFluidMoment(which, mom.mutable_data());
+            return mom;
           },
           py::arg("which"), "Flat AoS moments of ping-pong buffer `which` (0 current, 1 other).")
       .def(

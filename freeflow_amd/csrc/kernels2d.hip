@@ -172,14 +172,6 @@ __global__ void k_aos_to_soa(const float* __restrict__ aos, S* __restrict__ soa,
 #pragma unroll
   for (int q = 0; q < NM; q++) Store<S>::template store<DIM>(soa + q * plane + c, q, aos[c * NM + q], plane);
 }
-template <typename S, int DIM>
-__global__ void k_soa_to_aos(const S* __restrict__ soa, float* __restrict__ aos, long long n, size_t plane) {
-  constexpr int NM = DIM == 2 ? 6 : 10;
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= n) return;
-#pragma unroll
-  for (int q = 0; q < NM; q++) aos[c * NM + q] = Store<S>::template load<DIM>(soa + q * plane + c, q, plane);
-}
 
 // ---------------------------------------------------------------- initial state
 // initialize_state_kernel_2d/3d (LbmInitializer2D.cu:32-95,
@@ -297,21 +289,6 @@ int launch_convert_in(Domain& d, const float* aos, void* buf) {
 #define FF_CV(S)                                                                          \
   if (d.dim == 2) k_aos_to_soa<S, 2><<<g, b, 0, d.stream>>>(aos, (S*)buf, d.n, d.plane); \
   else k_aos_to_soa<S, 3><<<g, b, 0, d.stream>>>(aos, (S*)buf, d.n, d.plane);
-  if (d.storage == FF_STORAGE_F32) { FF_CV(float) }
-  else if (d.storage == FF_STORAGE_F16) { FF_CV(__half) }
-  else if (d.storage == FF_STORAGE_F16U) { FF_CV(h16u) }
-  else { FF_CV(__hip_bfloat16) }
-#undef FF_CV
-  FF_HIP(hipGetLastError());
-  return FF_OK;
-}
-
-int launch_convert_out(Domain& d, const void* buf, float* aos) {
-  const int b = 256;
-  const unsigned g = (unsigned)((d.n + b - 1) / b);
-#define FF_CV(S)                                                                                \
-  if (d.dim == 2) k_soa_to_aos<S, 2><<<g, b, 0, d.stream>>>((const S*)buf, aos, d.n, d.plane); \
-  else k_soa_to_aos<S, 3><<<g, b, 0, d.stream>>>((const S*)buf, aos, d.n, d.plane);
   if (d.storage == FF_STORAGE_F32) { FF_CV(float) }
   else if (d.storage == FF_STORAGE_F16) { FF_CV(__half) }
   else if (d.storage == FF_STORAGE_F16U) { FF_CV(h16u) }

@@ -582,11 +582,21 @@ void Simulator<D>::applyKinematicControl(int mesh_id, const std::vector<std::arr
 }
 
 template <int D>
-std::vector<float> Simulator<D>::getFluidMoment(int which) const {
+size_t Simulator<D>::fluidMomentCount() const {
   if (!m_dom) throw std::runtime_error("Simulator not initialized");
   const size_t n = (size_t)m_params.fluid_nx * m_params.fluid_ny * (D == 3 ? m_params.fluid_nz : 1);
-  std::vector<float> out(n * (D == 2 ? 6 : 10));
-  check(ff_get_moments(m_dom, out.data(), which), "ff_get_moments");
+  return n * (D == 2 ? 6 : 10);
+}
+
+template <int D>
+void Simulator<D>::readFluidMoment(int which, float* out) const {
+  check(ff_get_moments(m_dom, out, which), "ff_get_moments");
+}
+
+template <int D>
+std::vector<float> Simulator<D>::getFluidMoment(int which) const {
+  std::vector<float> out(fluidMomentCount());
+  readFluidMoment(which, out.data());
   return out;
 }
 

@@ -155,6 +155,8 @@ class Simulator {
   void saveFrameData(int frame_index, bool save_fluid, bool save_solid) const;
 
   std::vector<float> getFluidMoment(int which = 0) const;
+  size_t fluidMomentCount() const;  // floats of a moment buffer
+  void readFluidMoment(int which, float* out) const;
   std::vector<std::array<double, D>> getVertices() const;
   std::vector<std::array<double, D>> getVelocity() const;
   std::vector<std::array<double, D>> getForce() const;
