@@ -499,6 +499,7 @@ static int autotune(Batch& b) {
     FF_HIP(hipGetLastError());
     float ms = 0.f;
     FF_HIP(hipEventElapsedTime(&ms, e0, e1));
+    ms /= (float)iters;  // shapes of more cells per block repeat more often
     if (ms < best) {
       best = ms;
       best_t = t;
