@@ -20,7 +20,7 @@ LIB = os.path.join(PKG, "lib")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-HIP_SOURCES = ["capi.hip", "kernels2d.hip", "links.hip", "separable3d.hip", "readback.hip"]
+HIP_SOURCES = ["capi.hip", "kernels2d.hip", "links.hip", "separable3d.hip", "readback.hip", "rows3d.hip"]
 # compiled once per storage format (FF_TU_STORAGE): they instantiate every tile shape
 STORAGE_SOURCES = ["kernels3d.hip", "batch.hip"]
 

@@ -538,6 +538,7 @@ int ff_domain_create(const ff_domain_desc* desc, ff_domain** out) {
   const float cm = d.dim == 2 ? (float)(d.rho_f * d.dx * d.dx) : (float)(d.rho_f * d.dx * d.dx * d.dx);
   d.cf = (float)((double)cm * d.dx / (d.dt * d.dt));
   d.plane = plane_stride(n);
+  if (d.dim == 3) plan3d(d);
   d.h_flags.assign((size_t)n, kFluid);
   hipError_t e = acquire_stream(d.device, &d.stream);
   if (e != hipSuccess) { delete dd; return hip_fail(e, "hipStreamCreate"); }

@@ -98,6 +98,7 @@ struct Domain {
   int storage = FF_STORAGE_F32;
   unsigned options = 0;
   int tile2 = 0;     // 2D stream-collide tile shape (index into kTiles2)
+  int sep_chunks = 0, row_chunks = 0;  // z chunks of the whole-row 3D forms by the grid (plan3d)
   int tile3 = -1;    // 3D stream-collide tile shape (index into kTiles3), -1: by the grid
   double nu = 0, dx = 1, dt = 1, rho_f = 1;
   float nu_f = 0, cl = 1, ct = 1, cf = 1, omega = 1;
@@ -210,6 +211,8 @@ LinkArgs link_args(Domain& d, const float* v0, const float* v1, const float* u0,
 int launch_bulk2d(Domain& d, const void* in, void* out);
 int launch_bulk3d(Domain& d, const void* in, void* out);
 int launch_bulk3d_tiles(Domain& d, const void* in, void* out);
+int launch_rows3d(Domain& d, const void* in, void* out, int chunks);
+void plan3d(Domain& d);
 // boundary step: [detect] -> stream (tiles + boundary cells + next kinematics)
 // -> element sums + outlets + boundary-cell copy-back + next step's detection
 // -> finish (vertex forces, wrench)

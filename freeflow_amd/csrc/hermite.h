@@ -59,6 +59,15 @@ __device__ __forceinline__ bool is_wall3(uint8_t f) { return f < 12 && ((0xFE8u 
 // Fluid 1, SolidDynamic 4
 __device__ __forceinline__ bool is_updated(uint8_t f) { return f < 5 && ((0x12u >> f) & 1u); }
 
+// max(0, x), 0 for NaN: fmaxf(0, x) with one instruction.  The compiler adds a
+// second one to quiet a signalling NaN in a value that it has not seen
+// computed; populations are results of arithmetic, so there is none.
+__device__ __forceinline__ float clamp0(float x) {
+  float r;
+  asm("v_max_f32 %0, 0, %1" : "=v"(r) : "v"(x));
+  return r;
+}
+
 // Materialise an FP32 value in a register.  Without it the backend may fuse the
 // preceding multiply into a float->half conversion (v_fma_mix*), rounding the
 // exact product once to FP16 where the reference rounds to FP32 first.

@@ -202,6 +202,9 @@ __device__ __forceinline__ void sep_collide(const SepU& U, float omega, float* o
 // and stores exactly (behind a branch it had to wait for all of them).
 constexpr unsigned kNoCell = 0xFFFFFFFFu;
 using BufRsrc = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ BufRsrc buf_rsrc(const void* p) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)0xFFFFFFFF, 0x00027000);
+}
 
 __device__ __forceinline__ float sep_load(BufRsrc r, unsigned off, unsigned pb, int q) {
   return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)off, (int)(q * pb), 0));
@@ -264,7 +267,7 @@ inline int sep3d_plan(const Domain& d) {
   if (d.dim != 3 || d.storage != FF_STORAGE_F32 || !(d.options & FF_OPT_FAST_MATH) || (d.has_boundary && d.ne > 0) ||
       d.walls3)
     return 0;
-  return sep3d_chunks(d.nx, d.ny, d.nz, d.plane);
+  return d.sep_chunks;
 }
 
 template <bool PERIODIC>
@@ -283,9 +286,6 @@ __device__ __forceinline__ void sep3d_column(const float* __restrict__ in, float
   const unsigned pb = (unsigned)(plane * sizeof(float));  // bytes of a moment plane
   auto src_x = [&](int gx) { return PERIODIC ? ((gx % nx) + nx) % nx : min(nx - 1, max(0, gx)); };
   auto src_y = [&](int gy) { return PERIODIC ? ((gy % ny) + ny) % ny : min(ny - 1, max(0, gy)); };
-  auto rsrc = [&](const void* p) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)0xFFFFFFFF, 0x00027000);
-  };
   // Planes run from z0 - 1 to zend (one wrap at most); `i` counts them from 0,
   // past the last one it is taken again.
   const int np = zend - z0 + 2;
@@ -294,7 +294,7 @@ __device__ __forceinline__ void sep3d_column(const float* __restrict__ in, float
     return (unsigned)(PERIODIC ? (gz < 0 ? gz + nz : (gz >= nz ? gz - nz : gz)) : min(nz - 1, max(0, gz))) * nxy;
   };
   auto load = [&](int i, unsigned off, float* m) {
-    const BufRsrc r = rsrc(in + plane_at(i));
+    const BufRsrc r = buf_rsrc(in + plane_at(i));
 #pragma unroll
     for (int q = 0; q < 10; q++) m[q] = sep_load(r, off, pb, q);
   };
@@ -375,7 +375,7 @@ __device__ __forceinline__ void sep3d_column(const float* __restrict__ in, float
     // here let the wait for the moments at the top of every pass count them
     // out, the first pass included, instead of waiting for their write-back.
     auto put_results = [&](float* to_plane, unsigned to, const float* o) {
-      const BufRsrc r = rsrc(to_plane);
+      const BufRsrc r = buf_rsrc(to_plane);
 #pragma unroll
       for (int q = 0; q < 10; q++) sep_store(r, to, pb, q, o[q]);
     };
@@ -391,7 +391,7 @@ __device__ __forceinline__ void sep3d_column(const float* __restrict__ in, float
       const uint8_t fz = fl;
       row_stage(m, K, wave, hc, [&] {
         load(i + 1, src * sizeof(float), m);
-        fl = __builtin_amdgcn_raw_buffer_load_b8(rsrc(flags + plane_at(i + 1)), (int)cell, 0, 0);
+        fl = __builtin_amdgcn_raw_buffer_load_b8(buf_rsrc(flags + plane_at(i + 1)), (int)cell, 0, 0);
       });
       __syncthreads();
       // z stage of column k = (a', b') from its y moments t (c = 0, 1, 2):

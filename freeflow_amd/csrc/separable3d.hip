@@ -1,8 +1,9 @@
 // separable3d.hip -- 3D stream+collide launch of a domain stepped on its own:
-// the separable form (separable3d.h) where its rule says so, else the tiles
-// (kernels3d.hip).
+// the separable form (separable3d.h) or whole rows (rows3d.h) where their
+// rules say so, else the tiles (kernels3d.hip).
 
 #include "ff_internal.h"
+#include "rows3d.h"
 #include "separable3d.h"
 #include "stencil.h"
 
@@ -17,9 +18,17 @@ __global__ void __launch_bounds__(kSepThreads, 5)
   sep3d_tile<PERIODIC>(in, out, flags, nx, ny, nz, plane, omega, tiles_x, tiles_y, chunks, t);
 }
 
+void plan3d(Domain& d) {
+  d.sep_chunks = sep3d_chunks(d.nx, d.ny, d.nz, d.plane);
+  d.row_chunks = rows3d_chunks(d.nx, d.ny, d.nz, d.plane, storage_planes(d.storage, 3), storage_bytes(d.storage));
+}
+
 int launch_bulk3d(Domain& d, const void* in, void* out) {
   const int chunks = sep3d_plan(d);
-  if (!chunks) return launch_bulk3d_tiles(d, in, out);
+  if (!chunks) {
+    const int rows = rows3d_plan(d);
+    return rows ? launch_rows3d(d, in, out, rows) : launch_bulk3d_tiles(d, in, out);
+  }
   const int tx = (d.nx + kSepTX - 1) / kSepTX, ty = (d.ny + kSepTY - 1) / kSepTY, nt = tx * ty * chunks;
   const auto k = (d.options & FF_OPT_PERIODIC) ? k_sep3d<true> : k_sep3d<false>;
   launch_timed(k, dim3(xcd_grid(nt)), dim3(kSepThreads), d.stream, d.tev0, d.tev1, (const float*)in, (float*)out,
