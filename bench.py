@@ -58,11 +58,6 @@ METRIC = "MLUPS + % HBM peak; batched/served vs plain at ≤1e-3 rel err; p99 st
 HBM_PEAK_GBS = 8000.0
 # tile shapes by index, as in the library (ff_set_tile)
 TILES2 = ["32x8", "32x16", "64x8", "32x32", "64x16"]
-TILES3 = ["8x8x4 box", "16x4x4 box", "16x8 ring column x32", "16x8 ring column x16", "16x8 ring column x8",
-          "16x16 ring column x32", "16x16 ring column x16", "16x12 staged column x8", "16x26 staged column x8",
-          "64x4 staged column x16", "16x12 staged column x8, 2 planes in an LDS ring",
-          "16x8 staged column x8, 3 planes in an LDS ring", "32x8 staged column x8, 2 planes in an LDS ring",
-          "16x12 staged column x16, 3 planes in an LDS ring", "64x4 staged column x32", "32x12 staged column x16"]
 
 
 def bytes_per_lup(dim, storage_bytes, split_velocity=False):
@@ -122,10 +117,6 @@ def cpu_baseline_swimmer2d(state, budget_s=12.0):
 # (tx, ty, cells per thread) of the 2D tiles and (tx, ty, planes, kind, threads, planes in flight, LDS DMA)
 # of the 3D tiles, by tile index (ff_set_tile)
 SHAPES2 = [(32, 8, 1), (32, 8, 2), (64, 4, 2), (32, 8, 4), (64, 4, 4)]
-SHAPES3 = [(8, 8, 4, 0, 256, 1, 0), (16, 4, 4, 0, 256, 1, 0), (16, 8, 32, 1, 128, 1, 0), (16, 8, 16, 1, 128, 1, 0),
-           (16, 8, 8, 1, 128, 1, 0), (16, 16, 32, 1, 256, 1, 0), (16, 16, 16, 1, 256, 1, 0), (16, 12, 8, 2, 256, 1, 0),
-           (16, 26, 8, 2, 512, 1, 0), (64, 4, 16, 2, 448, 1, 0), (16, 12, 8, 2, 256, 2, 1), (16, 8, 8, 2, 192, 3, 1),
-           (32, 8, 8, 2, 384, 2, 1), (16, 12, 16, 2, 256, 3, 1), (64, 4, 32, 2, 448, 1, 0), (32, 12, 16, 2, 512, 1, 0)]
 
 
 def kernel2d(prefix, s, stage, periodic, tile, fast=False):
@@ -134,10 +125,12 @@ def kernel2d(prefix, s, stage, periodic, tile, fast=False):
             f"{str(fast and not stage).lower()}>")
 
 
-def kernel3d(s, periodic, tile, fast=False):
-    tx, ty, tz, kind, nt, pf, dma = SHAPES3[tile]
-    return (f"ff::k_bulk3d<{s}, {str(periodic).lower()}, {str(fast).lower()}, {kind}, {tx}, {ty}, {tz}, {nt}, {pf}, "
-            f"{str(bool(dma)).lower()}>")
+def kernel_rows3d(s, fast):
+    """The kernel that a periodic 256x128x128 domain without a body steps with
+    (whole 64-cell rows, whatever tile is set), and what to call its shape."""
+    if s == "float" and fast:
+        return "ff::k_sep3d<true>", "64x8 rows, moment space"
+    return f"ff::k_rows3d<{s}, true, {str(fast).lower()}>", "64x6 rows"
 
 
 def measured_traffic(kernel):
@@ -367,9 +360,10 @@ def tg3d_time(capi, wl, m, storage, fast, K, W, tile, tune=True):
     d.close()
     bpl = bytes_per_lup(3, 4 if storage == "f32" else 2, storage == "f16u")
     sname = {"f32": "float", "f16": "__half", "bf16": "__hip_bfloat16", "f16u": "ff::h16u"}[storage]
+    kernel, shape = kernel_rows3d(sname, fast)
     return {"mlups": cells * K / el / 1e6, "ms_per_step": el * 1e3 / K, "host_ms_per_step": host_el * 1e3 / K,
-            "tile": t, "avg_kernel_ms": avg_ms,
-            "kernel": kernel3d(sname, True, t, fast), "bytes_per_lup": bpl, "cells": cells,
+            "tile": t, "avg_kernel_ms": avg_ms, "shape": shape,
+            "kernel": kernel, "bytes_per_lup": bpl, "cells": cells,
             "frac": bpl * cells / (avg_ms * 1e-3) / (HBM_PEAK_GBS * 1e9), "mass_drift": drift, "steps": K + W}
 
 
@@ -502,7 +496,7 @@ def run_tg3d(args, capi, wl):
     forms = {("fast_math" if fast else "reference_order"): (st, fast, main_["tile"])}
 
     def summary(r):
-        return {"mlups": round(r["mlups"], 2), "ms_per_step": round(r["ms_per_step"], 5), "tile": TILES3[r["tile"]],
+        return {"mlups": round(r["mlups"], 2), "ms_per_step": round(r["ms_per_step"], 5), "tile": r["shape"],
                 "kernel": r["kernel"], "avg_kernel_us": round(r["avg_kernel_ms"] * 1e3, 3),
                 "bytes_per_lup": r["bytes_per_lup"], "frac": round(r["frac"], 4)}
     if st == "f32":
@@ -535,7 +529,7 @@ def run_tg3d(args, capi, wl):
     out = base_line(main_["mlups"], K, W, main_["ms_per_step"], f"f32 compute, {st} storage",
                     {"workload": f"3D D3Q27 {nx}x{ny}x{nz} Taylor-Green (amplitude 0.04) + vortex ring r=20, "
                                  "periodic, viscosity 0.01", "nx": nx, "ny": ny, "nz": nz, "storage": st,
-                     "arithmetic": arith, "tile": TILES3[main_["tile"]], "tile_index": main_["tile"],
+                     "arithmetic": arith, "tile": main_["shape"], "tile_index": main_["tile"],
                      "parallelism": "single-gpu"},
                     roof, cpu, mass_drift=main_["mass_drift"], **extra)
     print(json.dumps(out), flush=True)

@@ -245,7 +245,10 @@ int ff_domain_footprint(const ff_domain_desc* desc, int nv, int ne, const float*
    10-13 keep the next planes' moments in an LDS ring filled by LDS DMA with
    FP32 storage: 16x12 x 8 with 2 planes in flight, 16x8 x 8 with 3, 32x8 x 8
    with 2, 16x12 x 16 with 3; 14: 64x4 x 32, 15: 32x12 x 16).
-   0 is the default; results do not depend on it (in either arithmetic form).
+   A 2D domain that was neither set nor tuned takes 0, a 3D one a shape by its
+   grid.  3D domains without a body and bounce-back walls step with whole-row
+   kernels instead where their grid fills the chip with them, whatever is set
+   here.  Results do not depend on the shape (in either arithmetic form).
    No counterpart in the reference (its tile is fixed, CudaCommon.cuh:44-51). */
 int ff_set_tile(ff_domain* d, int tile);
 /* Time every tile shape on this domain (three interleaved rounds, each
