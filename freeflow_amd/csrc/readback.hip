@@ -87,6 +87,21 @@ struct Pinned {
   }
 };
 
+// Waits for the stream on every way out, errors too, before a block declared
+// above it is lent again: kernels queued by a call that fails later still
+// write the block.
+struct StreamWait {
+  const hipStream_t stream;
+  bool done = false;
+  hipError_t wait() {
+    done = true;
+    return hipStreamSynchronize(stream);
+  }
+  ~StreamWait() {
+    if (!done) (void)hipStreamSynchronize(stream);
+  }
+};
+
 // Small pinned pieces that live as long as their owner, cut from shared slabs
 // (a pinned allocation of its own costs a domain 50-65 us).  A slab is given
 // back when its last piece is freed; one empty slab is kept while a domain
@@ -159,9 +174,10 @@ int read_spans(Domain& d, const Span* spans, int n) {
   if (words * 4 <= kPinnedBytes[0]) {
     Pinned b(0);
     if (b.p) {
+      StreamWait queued{d.stream};
       k_gather<<<(unsigned)std::min<size_t>(32, (largest + 255) / 256), 256, 0, d.stream>>>(a, (uint32_t*)b.p);
       FF_HIP(hipGetLastError());
-      FF_HIP(hipStreamSynchronize(d.stream));
+      FF_HIP(queued.wait());
       for (int s = 0; s < n; s++)
         if (spans[s].bytes) std::memcpy(spans[s].host, b.p + (size_t)a.off[s] * 4, spans[s].bytes);
       return FF_OK;
@@ -177,8 +193,9 @@ int read_kernel_output(Domain& d, size_t bytes, void* out, int (*launch)(Domain&
   if (bytes <= kPinnedBytes[0]) {
     Pinned b(0);
     if (b.p) {
+      StreamWait queued{d.stream};
       if (int rc = launch(d, b.p)) return rc;
-      FF_HIP(hipStreamSynchronize(d.stream));
+      FF_HIP(queued.wait());
       std::memcpy(out, b.p, bytes);
       return FF_OK;
     }
