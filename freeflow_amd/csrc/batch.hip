@@ -65,7 +65,7 @@ struct Batch {
   bool dirty = true;
   int tile = -1;        // fixed tile shape (index into kTiles2 / kTiles3), -1 = autotune
   int tuned_tile = -1;  // result of the last tile search
-  double tuned_cells = 0.0;  // member cells when the search ran (a change by 2x searches again)
+  double tuned_cells = 0.0;  // cells in tiles when the search ran (a change by 2x searches again)
   DomDev* d_doms = nullptr;
   size_t doms_cap = 0;
   int2* d_map = nullptr;
@@ -458,9 +458,11 @@ static int build_tables(Batch& b, int tile) {
   return FF_OK;
 }
 
-static double member_cells(const Batch& b) {
+// Cells of the members that step with tiles.
+static double tiled_cells(const Batch& b) {
   double c = 0.0;
-  for (const Domain* d : b.mem) c += (double)d->nx * d->ny * d->nz;
+  for (const Domain* d : b.mem)
+    if (!sep3d_plan(*d)) c += (double)d->nx * d->ny * d->nz;
   return c;
 }
 
@@ -470,13 +472,9 @@ static double member_cells(const Batch& b) {
 // table build and a few launches of the whole batch while a server waits).
 constexpr int kBatchCand3[] = {0, 7, 8, 9, 14, 15};
 
-// Time the stream-collide tiles of every member for each candidate shape
-// and keep the fastest.
+// Time the stream-collide tiles of every member that has them for each
+// candidate shape and keep the fastest.
 static int autotune(Batch& b) {
-  if (b.mem.empty()) {
-    b.tuned_tile = 0;
-    return FF_OK;
-  }
   const int ncand = b.dim == 2 ? kNumTiles2 : (int)(sizeof(kBatchCand3) / sizeof(kBatchCand3[0]));
   EventSet ev;
   FF_HIP(ev.create(2));
@@ -506,7 +504,7 @@ static int autotune(Batch& b) {
     }
   }
   b.tuned_tile = best_t;
-  b.tuned_cells = member_cells(b);
+  b.tuned_cells = tiled_cells(b);
   return rc;
 }
 
@@ -578,9 +576,11 @@ static int rebuild(Batch& b) {
   drop_graph(b);
   int rc;
   // the best tile depends on how many blocks the launch holds: search again
-  // when the member cells changed by more than 2x since the last search
-  const double cells = member_cells(b);
-  const bool retune = b.tuned_tile < 0 || cells > 2.0 * b.tuned_cells || 2.0 * cells < b.tuned_cells;
+  // when the cells in tiles changed by more than 2x since the last search;
+  // with none there is nothing to time
+  const double cells = tiled_cells(b);
+  const bool retune =
+      cells > 0.0 && (b.tuned_tile < 0 || cells > 2.0 * b.tuned_cells || 2.0 * cells < b.tuned_cells);
   if (b.tile < 0 && retune && (rc = autotune(b))) return rc;
   if ((rc = build_tables(b, current_tile(b)))) return rc;
   b.direct = 0;  // the graphs are captured on demand (replay)
