@@ -58,6 +58,11 @@ METRIC = "MLUPS + % HBM peak; batched/served vs plain at ≤1e-3 rel err; p99 st
 HBM_PEAK_GBS = 8000.0
 # tile shapes by index, as in the library (ff_set_tile)
 TILES2 = ["32x8", "32x16", "64x8", "32x32", "64x16"]
+TILES3 = ["8x8x4 box", "16x4x4 box", "16x8 ring column x32", "16x8 ring column x16", "16x8 ring column x8",
+          "16x16 ring column x32", "16x16 ring column x16", "16x12 staged column x8", "16x26 staged column x8",
+          "64x4 staged column x16", "16x12 staged column x8, 2 planes in an LDS ring",
+          "16x8 staged column x8, 3 planes in an LDS ring", "32x8 staged column x8, 2 planes in an LDS ring",
+          "16x12 staged column x16, 3 planes in an LDS ring", "64x4 staged column x32", "32x12 staged column x16"]
 
 
 def bytes_per_lup(dim, storage_bytes, split_velocity=False):
@@ -117,6 +122,10 @@ def cpu_baseline_swimmer2d(state, budget_s=12.0):
 # (tx, ty, cells per thread) of the 2D tiles and (tx, ty, planes, kind, threads, planes in flight, LDS DMA)
 # of the 3D tiles, by tile index (ff_set_tile)
 SHAPES2 = [(32, 8, 1), (32, 8, 2), (64, 4, 2), (32, 8, 4), (64, 4, 4)]
+SHAPES3 = [(8, 8, 4, 0, 256, 1, 0), (16, 4, 4, 0, 256, 1, 0), (16, 8, 32, 1, 128, 1, 0), (16, 8, 16, 1, 128, 1, 0),
+           (16, 8, 8, 1, 128, 1, 0), (16, 16, 32, 1, 256, 1, 0), (16, 16, 16, 1, 256, 1, 0), (16, 12, 8, 2, 256, 1, 0),
+           (16, 26, 8, 2, 512, 1, 0), (64, 4, 16, 2, 448, 1, 0), (16, 12, 8, 2, 256, 2, 1), (16, 8, 8, 2, 192, 3, 1),
+           (32, 8, 8, 2, 384, 2, 1), (16, 12, 16, 2, 256, 3, 1), (64, 4, 32, 2, 448, 1, 0), (32, 12, 16, 2, 512, 1, 0)]
 
 
 def kernel2d(prefix, s, stage, periodic, tile, fast=False):
@@ -125,12 +134,16 @@ def kernel2d(prefix, s, stage, periodic, tile, fast=False):
             f"{str(fast and not stage).lower()}>")
 
 
-def kernel_rows3d(s, fast):
-    """The kernel that a periodic 256x128x128 domain without a body steps with
-    (whole 64-cell rows, whatever tile is set), and what to call its shape."""
-    if s == "float" and fast:
+def kernel3d(capi, s, form, tile, fast):
+    """The kernel that a periodic 3D domain without a body steps with in a
+    form and tile of Domain.tile(), and what to call its shape."""
+    if form == capi.FORM_SEPARABLE:
         return "ff::k_sep3d<true>", "64x8 rows, moment space"
-    return f"ff::k_rows3d<{s}, true, {str(fast).lower()}>", "64x6 rows"
+    if form == capi.FORM_ROWS:
+        return f"ff::k_rows3d<{s}, true, {str(fast).lower()}>", "64x6 rows"
+    tx, ty, tz, kind, nt, pf, dma = SHAPES3[tile]
+    return (f"ff::k_bulk3d<{s}, true, {str(fast).lower()}, {kind}, {tx}, {ty}, {tz}, {nt}, {pf}, "
+            f"{str(bool(dma)).lower()}>", TILES3[tile])
 
 
 def measured_traffic(kernel):
@@ -332,7 +345,8 @@ def run_batched(args, capi, wl):
 
 def tg3d_time(capi, wl, m, storage, fast, K, W, tile, tune=True):
     """Time K steps of the 3D workload (after W warm-up steps) in one form;
-    returns the rate, the chosen tile and the stream-collide launch time."""
+    returns the rate, the tile it stepped with (None: whole rows) and the
+    stream-collide launch time."""
     c = wl.TG3D
     nx, ny, nz = c["nx"], c["ny"], c["nz"]
     cells = nx * ny * nz
@@ -340,13 +354,15 @@ def tg3d_time(capi, wl, m, storage, fast, K, W, tile, tune=True):
     d.set_moments(m)
     if tile >= 0:
         d.set_tile(tile)
-        t = tile
-    else:
-        t = d.autotune() if tune else 0
+    elif tune:
+        d.autotune()
+    sname = {"f32": "float", "f16": "__half", "bf16": "__hip_bfloat16", "f16u": "ff::h16u"}[storage]
+    form, t = d.tile()
+    kernel, shape = kernel3d(capi, sname, form, t, fast)
     m0 = d.mass()
     d.step(W)
     d.sync()
-    print(f"[bench] tg3d {storage} {'fast' if fast else 'reference-order'} tile {t}: timing {K} steps",
+    print(f"[bench] tg3d {storage} {'fast' if fast else 'reference-order'}, {shape}: timing {K} steps",
           file=sys.stderr, flush=True)
     # the timed region: K steps, each step's stream launch timed by HIP events
     # attached to the launch (the kernel as stepping runs it: each launch reads
@@ -359,10 +375,8 @@ def tg3d_time(capi, wl, m, storage, fast, K, W, tile, tune=True):
     drift = abs(d.mass() - m0) / m0
     d.close()
     bpl = bytes_per_lup(3, 4 if storage == "f32" else 2, storage == "f16u")
-    sname = {"f32": "float", "f16": "__half", "bf16": "__hip_bfloat16", "f16u": "ff::h16u"}[storage]
-    kernel, shape = kernel_rows3d(sname, fast)
     return {"mlups": cells * K / el / 1e6, "ms_per_step": el * 1e3 / K, "host_ms_per_step": host_el * 1e3 / K,
-            "tile": t, "avg_kernel_ms": avg_ms, "shape": shape,
+            "tile": t if form == capi.FORM_TILES else None, "avg_kernel_ms": avg_ms, "shape": shape,
             "kernel": kernel, "bytes_per_lup": bpl, "cells": cells,
             "frac": bpl * cells / (avg_ms * 1e-3) / (HBM_PEAK_GBS * 1e9), "mass_drift": drift, "steps": K + W}
 
@@ -371,7 +385,7 @@ def cpu_baseline_tg3d(capi, wl, m, steps, forms):
     """CPU leg of the 3D workload: the FP32 CPU oracle (OpenMP, timed: the
     cpu_baseline) and the FP64 oracle, `steps` steps on the full grid from
     the same state, against the GPU forms timed (`forms`: name -> (storage,
-    fast math, tile))."""
+    fast math, tile or None))."""
     sys.path.insert(0, os.path.join(ROOT, "tests"))
     import oracle_lib as ol
     c = wl.TG3D
@@ -382,7 +396,8 @@ def cpu_baseline_tg3d(capi, wl, m, steps, forms):
     gpu = {}
     for name, (storage, fast, tile) in forms.items():
         d = capi.Domain(3, nx, ny, nz, viscosity=c["viscosity"], storage=storage, periodic=True, fast_math=fast)
-        d.set_tile(tile)
+        if tile is not None:
+            d.set_tile(tile)
         d.set_moments(m32)
         d.step(steps)
         gpu[name] = d.moments(0).astype(np.float64)
@@ -529,7 +544,8 @@ def run_tg3d(args, capi, wl):
     out = base_line(main_["mlups"], K, W, main_["ms_per_step"], f"f32 compute, {st} storage",
                     {"workload": f"3D D3Q27 {nx}x{ny}x{nz} Taylor-Green (amplitude 0.04) + vortex ring r=20, "
                                  "periodic, viscosity 0.01", "nx": nx, "ny": ny, "nz": nz, "storage": st,
-                     "arithmetic": arith, "tile": main_["shape"], "tile_index": main_["tile"],
+                     "arithmetic": arith, "tile": main_["shape"],
+                     **({} if main_["tile"] is None else {"tile_index": main_["tile"]}),
                      "parallelism": "single-gpu"},
                     roof, cpu, mass_drift=main_["mass_drift"], **extra)
     print(json.dumps(out), flush=True)

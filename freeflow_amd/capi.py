@@ -19,6 +19,7 @@ STORAGE = {"f32": 0, "f16": 1, "bf16": 2, "f16u": 3}
 OPT_STAGE_FP16 = 0x1
 OPT_PERIODIC = 0x2
 OPT_FAST_MATH = 0x4
+FORM_TILES, FORM_ROWS, FORM_SEPARABLE = 0, 1, 2
 
 # fsi::lbm::LbmNodeFlag ordinals (LbmDataTypes.cuh:17-56)
 FLAG = {
@@ -33,7 +34,8 @@ EXPORTS = [
     "ff_get_moments", "ff_set_boundary", "ff_update_boundary", "ff_set_body_ref", "ff_set_wave", "ff_set_wave_params", "ff_step",
     "ff_step_proxy", "ff_get_vertex_forces", "ff_get_step_vertex_forces", "ff_get_step_vertex_forces_noalloc", "ff_get_body_wrench", "ff_set_wrench_history",
     "ff_get_wrench_history", "ff_get_body_power", "ff_get_power_history", "ff_get_boundary", "ff_mass", "ff_fill_solid", "ff_sync", "ff_time_bulk_kernel",
-    "ff_time_steps", "ff_step_timed", "ff_domain_footprint", "ff_set_tile", "ff_autotune", "ff_batch_create", "ff_batch_destroy", "ff_batch_add",
+    "ff_time_steps", "ff_step_timed", "ff_domain_footprint", "ff_set_tile", "ff_get_tile", "ff_autotune",
+    "ff_batch_create", "ff_batch_destroy", "ff_batch_add",
     "ff_batch_remove", "ff_batch_size", "ff_batch_step", "ff_batch_sync", "ff_batch_set_tile", "ff_batch_get_tile",
     "ff_batch_time_steps", "ff_batch_time_bulk", "ff_last_error", "ff_device_count", "ff_version",
 ]
@@ -95,6 +97,7 @@ def lib():
         L.ff_device_count.argtypes = [C.POINTER(C.c_int)]
         L.ff_domain_footprint.argtypes = [C.POINTER(DomainDesc), C.c_int, C.c_int, vp, vp, C.POINTER(C.c_ulonglong)]
         L.ff_set_tile.argtypes = [vp, C.c_int]
+        L.ff_get_tile.argtypes = [vp, C.POINTER(C.c_int), C.POINTER(C.c_int)]
         L.ff_autotune.argtypes = [vp, C.POINTER(C.c_int)]
         L.ff_batch_create.argtypes = [C.c_int, C.c_int, C.c_uint, C.c_int, C.POINTER(vp)]
         L.ff_batch_destroy.argtypes = [vp]
@@ -307,6 +310,13 @@ class Domain:
 
     def set_tile(self, tile):
         _check(lib().ff_set_tile(self.h, tile))
+
+    def tile(self):
+        """(form, tile) of the next step: FORM_TILES, FORM_ROWS or
+        FORM_SEPARABLE, and the shape it takes where it steps with tiles."""
+        f, t = C.c_int(0), C.c_int(0)
+        _check(lib().ff_get_tile(self.h, C.byref(f), C.byref(t)))
+        return f.value, t.value
 
     def autotune(self):
         t = C.c_int(0)

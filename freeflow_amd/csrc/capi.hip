@@ -1158,7 +1158,15 @@ int ff_set_tile(ff_domain* dd, int tile) {
   if (tile < 0 || tile >= n) return fail(FF_ERR_INVALID, "tile index out of range");
   if (dd->dim == 2) dd->tile2 = tile;
   else dd->tile3 = tile;
+  dd->rows3 = false;
   batch_mark_dirty(dd->batch);
+  return FF_OK;
+}
+
+int ff_get_tile(ff_domain* dd, int* form, int* tile) {
+  FF_CHECK_DOMAIN(dd);
+  if (!form || !tile) return fail(FF_ERR_INVALID, "null output");
+  *form = stream_form(*dd, tile);
   return FF_OK;
 }
 
@@ -1167,6 +1175,11 @@ int ff_autotune(ff_domain* dd, int* tile) {
   Domain& d = *dd;
   if (d.batch) return fail(FF_ERR_STATE, "domain belongs to a batch: its tile is tuned with the batch");
   FF_HIP(hipSetDevice(d.device));
+  int now = 0;
+  if (stream_form(d, &now) == FF_FORM_SEPARABLE) {  // whatever tile it has
+    if (tile) *tile = now;
+    return FF_OK;
+  }
   EventSet ev;
   FF_HIP(ev.create(2));
   const hipEvent_t e0 = ev[0], e1 = ev[1];
@@ -1177,23 +1190,28 @@ int ff_autotune(ff_domain* dd, int* tile) {
   int rc = FF_OK;
   int& cur = d.dim == 2 ? d.tile2 : d.tile3;
   const int n = d.dim == 2 ? kNumTiles2 : kNumTiles3;
-  const int saved = cur;
   // an error return leaves the tile the domain had
   struct Restore {
-    int& t;
-    int v;
-    bool keep = false;
+    Domain& d;
+    int t2 = d.tile2, t3 = d.tile3;
+    bool rows = d.rows3, keep = false;
     ~Restore() {
-      if (!keep) t = v;
+      if (keep) return;
+      d.tile2 = t2;
+      d.tile3 = t3;
+      d.rows3 = rows;
     }
-  } restore{cur, saved};
-  auto launch = [&]() { return d.dim == 2 ? launch_bulk2d(d, in, out) : launch_bulk3d_tiles(d, in, out); };
+  } restore{d};
+  d.rows3 = true;
+  const bool rows = stream_form(d, &now) == FF_FORM_ROWS;  // the last candidate: the same bits as the tiles
+  auto launch = [&]() { return d.dim == 2 ? launch_bulk2d(d, in, out) : launch_bulk3d(d, in, out); };
   // rounds over every candidate (clock and cache drift hit all alike); each
   // candidate keeps its fastest round
-  std::vector<double> best(n, 1e30);
+  std::vector<double> best(n + (rows ? 1 : 0), 1e30);
   for (int round = 0; round < 3 && !rc; round++) {
-    for (int t = 0; t < n && !rc; t++) {
-      cur = t;
+    for (int t = 0; t < (int)best.size() && !rc; t++) {
+      if (t < n) cur = t;
+      d.rows3 = t == n;
       for (int w = 0; w < 3 && !rc; w++) rc = launch();
       if (rc) break;
       FF_HIP(hipEventRecord(e0, d.stream));
@@ -1205,11 +1223,12 @@ int ff_autotune(ff_domain* dd, int* tile) {
       best[t] = std::min(best[t], (double)ms);
     }
   }
-  const int best_t = (int)(std::min_element(best.begin(), best.end()) - best.begin());
-  cur = rc ? saved : best_t;
+  if (rc) return rc;
+  cur = (int)(std::min_element(best.begin(), best.begin() + n) - best.begin());
+  d.rows3 = rows && best[n] < best[cur];
   restore.keep = true;
-  if (tile) *tile = std::max(cur, 0);
-  return rc;
+  if (tile) *tile = cur;
+  return FF_OK;
 }
 
 }  // extern "C"

@@ -100,6 +100,7 @@ struct Domain {
   int tile2 = 0;     // 2D stream-collide tile shape (index into kTiles2)
   int sep_chunks = 0, row_chunks = 0;  // z chunks of the whole-row 3D forms by the grid (plan3d)
   int tile3 = -1;    // 3D stream-collide tile shape (index into kTiles3), -1: by the grid
+  bool rows3 = true;  // whole rows in place of tiles where row_chunks says so: not for a tile set or tuned faster
   double nu = 0, dx = 1, dt = 1, rho_f = 1;
   float nu_f = 0, cl = 1, ct = 1, cf = 1, omega = 1;
   size_t plane = 0;  // elements between moment planes
@@ -213,6 +214,8 @@ int launch_bulk3d(Domain& d, const void* in, void* out);
 int launch_bulk3d_tiles(Domain& d, const void* in, void* out);
 int launch_rows3d(Domain& d, const void* in, void* out, int chunks);
 void plan3d(Domain& d);
+int tile3_of(const Domain& d, bool body);
+int stream_form(const Domain& d, int* tile);
 // boundary step: [detect] -> stream (tiles + boundary cells + next kinematics)
 // -> element sums + outlets + boundary-cell copy-back + next step's detection
 // -> finish (vertex forces, wrench)

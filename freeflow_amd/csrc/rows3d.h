@@ -52,7 +52,7 @@ inline int rows3d_chunks(int nx, int ny, int nz, size_t plane, size_t planes, si
 }
 
 inline int rows3d_plan(const Domain& d) {
-  if (d.dim != 3 || (d.has_boundary && d.ne > 0) || d.walls3) return 0;
+  if (d.dim != 3 || !d.rows3 || (d.has_boundary && d.ne > 0) || d.walls3) return 0;
   return d.row_chunks;
 }
 

@@ -23,6 +23,17 @@ void plan3d(Domain& d) {
   d.row_chunks = rows3d_chunks(d.nx, d.ny, d.nz, d.plane, storage_planes(d.storage, 3), storage_bytes(d.storage));
 }
 
+// The form of the domain's next step (FF_FORM_*) and the tile that it takes
+// where it has tiles.
+int stream_form(const Domain& d, int* tile) {
+  if (d.dim == 2) {
+    *tile = d.tile2;
+    return FF_FORM_TILES;
+  }
+  *tile = tile3_of(d, d.has_boundary && d.ne > 0);
+  return sep3d_plan(d) ? FF_FORM_SEPARABLE : (rows3d_plan(d) ? FF_FORM_ROWS : FF_FORM_TILES);
+}
+
 int launch_bulk3d(Domain& d, const void* in, void* out) {
   const int chunks = sep3d_plan(d);
   if (!chunks) {

@@ -246,15 +246,28 @@ int ff_domain_footprint(const ff_domain_desc* desc, int nv, int ne, const float*
    FP32 storage: 16x12 x 8 with 2 planes in flight, 16x8 x 8 with 3, 32x8 x 8
    with 2, 16x12 x 16 with 3; 14: 64x4 x 32, 15: 32x12 x 16).
    A 2D domain that was neither set nor tuned takes 0, a 3D one a shape by its
-   grid.  3D domains without a body and bounce-back walls step with whole-row
-   kernels instead where their grid fills the chip with them, whatever is set
-   here.  Results do not depend on the shape (in either arithmetic form).
+   grid, or whole rows (below) where its grid fills the chip with them.
+   Results do not depend on the shape (in either arithmetic form).
    No counterpart in the reference (its tile is fixed, CudaCommon.cuh:44-51). */
 int ff_set_tile(ff_domain* d, int tile);
 /* Time every tile shape on this domain (three interleaved rounds, each
    shape's best round; the state is left unchanged) and keep the fastest;
-   writes its index to *tile. */
+   writes its index to *tile.  Where whole rows serve they are timed too, and
+   kept if they are faster than that shape.  A domain that steps with the
+   separable form has no shape to choose: *tile is the one of ff_get_tile. */
 int ff_autotune(ff_domain* d, int* tile);
+/* How the next step runs the domain's cells: *form is one of FF_FORM_*, *tile
+   the shape it takes where it steps with tiles.
+   Whole rows (64 x 6 cells marching along z, the bits of the tiles): 3D
+   domains without a body and bounce-back walls, unless a tile was set or was
+   the faster one when tuned.  Separable (64 x 8 cells in moment space, its own
+   rounding): such domains with FP32 storage and FF_OPT_FAST_MATH, by their
+   grid alone, whatever tile is set.  Members of a batch take the tile of the
+   batch for either of the first two. */
+#define FF_FORM_TILES 0
+#define FF_FORM_ROWS 1
+#define FF_FORM_SEPARABLE 2
+int ff_get_tile(ff_domain* d, int* form, int* tile);
 
 /* ---- batches: many domains of one kind stepped together ----------------
    No counterpart in the reference, which steps one flow field per Simulator
