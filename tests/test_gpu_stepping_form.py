@@ -1,10 +1,13 @@
 """Which kernel a 3D domain steps with (Domain.tile): a tile that the caller
 sets is the one that runs wherever the results do not depend on it, tuning
 keeps whole rows only where they serve, and the separable form is by the grid
-alone."""
+alone.  The tests of the whole-row kernels reach them on the grids that they
+name; the columns keep a full-grid comparison in both arithmetic forms."""
 import numpy as np
 import pytest
 
+import oracle_lib as ol
+import test_gpu_rows3d as rows
 import test_gpu_separable3d as sep
 from freeflow_amd import capi, workloads as wl
 
@@ -70,3 +73,67 @@ def test_separable_form_is_by_the_grid():
     assert a.tile()[0] == capi.FORM_TILES
     for x in (a, b):
         x.close()
+
+
+def test_grids_of_the_whole_row_tests_reach_them():
+    for grids, want, kw in ((rows.GRIDS, capi.FORM_ROWS, [dict(storage=s, fast_math=f) for s, f in
+                                                          [("f32", False), ("f16", True), ("f16", False), ("bf16", True),
+                                                           ("f16u", True), ("f16u", False)]]),
+                            (sep.GRIDS + [(127, 50, 90)], capi.FORM_SEPARABLE, [dict(fast_math=True)])):
+        for g in grids:
+            for k in kw:
+                for periodic in (True, False):
+                    d = capi.Domain(3, *g, viscosity=0.02, periodic=periodic, **k)
+                    assert d.tile()[0] == want, (g, k)
+                    d.close()
+
+
+@pytest.mark.parametrize("grid", [(276, 201, 10), (277, 202, 86)])
+@pytest.mark.parametrize("periodic", [True, False])
+def test_fast_fp32_rows_equal_columns(grid, periodic):
+    """Grids whose rows serve where the separable form does not."""
+    print(f"case fast rows {grid} periodic={periodic}", flush=True)
+    m, f = rows.setup(grid, 9, periodic)
+    d = [capi.Domain(3, *grid, viscosity=0.02, periodic=periodic, fast_math=True) for _ in range(2)]
+    for x in d:
+        x.set_flags(f)
+        x.set_moments(m)
+    d[1].set_tile(7)
+    assert [x.tile()[0] for x in d] == [capi.FORM_ROWS, capi.FORM_TILES]
+    for x in d:
+        x.step(5)
+    assert np.array_equal(d[0].moments(0), d[1].moments(0))
+    for x in d:
+        x.close()
+
+
+def test_columns_on_a_full_grid_with_a_wall():
+    """The 64x4 columns in both forms on 256x128x128 with a wall and a block
+    of wall cells, against the FP32 oracle; the fast form within the 1e-5
+    relative L2 that it is held to elsewhere."""
+    c = wl.TG3D
+    grid = (c["nx"], c["ny"], c["nz"])
+    print(f"case columns {grid} with a wall", flush=True)
+    m = np.asarray(wl.taylor_green_ring(*grid, c["amp"], c["ring_r"], c["seed"]), np.float32)
+    f = np.ones(grid[::-1], np.uint8)
+    f[:, 0, :] = 5
+    f[60:64, 50:55, 100:107] = 3
+    ol.set_threads(0)
+    o = ol.OracleDomain(3, *grid, fp64=False, stage_fp16=False, periodic=True, nu=c["viscosity"])
+    o.set_flags(f.ravel())
+    o.set_moments(m.astype(np.float64))
+    o.step(20)
+    ref = o.moments(0)
+    for fast in (False, True):
+        d = capi.Domain(3, *grid, viscosity=c["viscosity"], periodic=True, fast_math=fast)
+        d.set_flags(f.ravel())
+        d.set_tile(9)
+        assert d.tile() == (capi.FORM_TILES, 9)
+        d.set_moments(m)
+        d.step(20)
+        got = d.moments(0).astype(np.float64)
+        d.close()
+        if fast:
+            assert np.linalg.norm(got - ref) <= 1e-5 * np.linalg.norm(ref)
+        else:
+            assert np.array_equal(got, ref)
