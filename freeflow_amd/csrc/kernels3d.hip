@@ -11,6 +11,7 @@
 
 #include "ff_internal.h"
 #include "links_body.h"
+#include "plan3d.h"
 #include "stencil.h"
 
 namespace ff {
@@ -111,28 +112,9 @@ template int step3d_typed<tu_storage>(Domain&, const void*, void*, const LinkArg
 template int bulk3d_typed<tu_storage>(Domain&, const void*, void*);
 
 #if FF_TU_STORAGE == 0
-// Tile of a domain whose tile was neither set nor tuned; any tile gives the
-// same results.  us a step (FP32 reference order / fast):
-//   box 8x8x4: few cells fill the chip only in small boxes.  64^3 16.6 / 13.1
-//   against 29.9 / 25.1 of the 16x12x8 column, 80^3 28.4 / 24.8 against
-//   33.7 / 28.9, 96x96x64 32.9 / 28.9 against 34.1 / 28.5; at 203x101x97
-//   104 / 90 against 66 / 56.  With a body the launch waits for its boundary
-//   cells too: 64^3 23.3 / 22.1 against 25.0 / 20.8, 96x64x64 30.4 / 27.8
-//   against 30.2 / 24.1, 160x96x96 84.7 / 73.6 against 56.1 / 45.0.
-//   column 16x12x8 in between.
-//   column 32x12x16 once both moment buffers exceed the last-level cache, so
-//   that halo cells are read from memory again, and if its tiles are not
-//   padding for more than a fifth: 256x192x160 189 / 177 against 229 / 224
-//   (FP16 148 against 153), 384x256x256 650 / 622 against 811 / 807, but
-//   100x300x200 (33 % padding) 216 / 198 against 194 / 191, and FP16
-//   250x150x150 (225 MB) 126 against 103.
 int tile3_of(const Domain& d, bool body) {
   if (d.tile3 >= 0) return d.tile3;
-  const long long n = (long long)d.nx * d.ny * d.nz;
-  if (n < (body ? 350000 : 580000)) return 0;
-  const double bytes = 2.0 * (double)d.plane * storage_planes(d.storage, 3) * storage_bytes(d.storage);
-  const long long padded = (long long)((d.nx + 31) / 32 * 32) * ((d.ny + 11) / 12 * 12) * ((d.nz + 15) / 16 * 16);
-  return bytes > 256e6 && 5 * padded < 6 * n ? 15 : 7;
+  return default_tile3({d.nx, d.ny, d.nz}, d.plane, storage_planes(d.storage, 3), storage_bytes(d.storage), body);
 }
 
 #define FF_ELSEWHERE(S)                                                                                          \

@@ -26,31 +26,9 @@ namespace ff {
 // 256x192x160: FP16 fast 147 -> 113 us (split velocity 177 -> 139), FP32
 // reference order 189 -> 163; 250x150x150: 102 -> 78, 144 -> 110, 173 -> 141.
 // Rows of 8 (96 VGPRs, 5 spilled) 146 us in FP16.
-constexpr int kRowsTX = 64, kRowsTY = 6;
 constexpr int kRowsThreads = 64 * (kRowsTY + 2);
 
-// Number of z chunks of the rows for a grid, or 0 where the columns are
-// faster.  512 blocks share the chip and a chunk of n planes takes n + 2 plane
-// steps; a step takes as long as about 100 blocks of the 16x12x8 column (2.6 us
-// and 0.027 us a block in FP16 fast, 3.9 and 0.040 in FP32 reference order):
-// 51 us against 48 at 203x101x97, 33 against 31 at 160x96x96 (padding to 64
-// cells), 69 against 75 at 256x128x128.  Buffers beyond 4 GiB take the columns.
-inline int rows3d_chunks(int nx, int ny, int nz, size_t plane, size_t planes, size_t elem) {
-  if ((plane * planes + (size_t)nx * ny) * elem >= 0xFFFF0000ull) return 0;
-  const long long cols = (long long)((nx + kRowsTX - 1) / kRowsTX) * ((ny + kRowsTY - 1) / kRowsTY);
-  long long best = 0;
-  int chunks = 0;
-  for (int c = 1; c <= nz; c++) {
-    const long long cost = ((nz + c - 1) / c + 2) * ((cols * c + 511) / 512);
-    if (!chunks || cost < best) {
-      best = cost;
-      chunks = c;
-    }
-  }
-  const long long tiles = (long long)((nx + 15) / 16) * ((ny + 11) / 12) * ((nz + 7) / 8);
-  return 100 * best < tiles ? chunks : 0;
-}
-
+// The domain's whole rows: their z chunks, or 0 if it steps with the tiles.
 inline int rows3d_plan(const Domain& d) {
   if (d.dim != 3 || !d.rows3 || (d.has_boundary && d.ne > 0) || d.walls3) return 0;
   return d.row_chunks;

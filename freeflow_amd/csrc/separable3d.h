@@ -24,6 +24,7 @@
 
 #include "ff_internal.h"
 #include "hermite.h"
+#include "plan3d.h"
 
 namespace ff {
 
@@ -228,33 +229,8 @@ __device__ __forceinline__ void sep_store(BufRsrc r, unsigned off, unsigned pb, 
 // rows of 4 or 6 (91-97 us), non-temporal loads (halo rows miss L2: 97-106 us),
 // stores a plane later (no change once their count is exact), the side columns
 // of three planes at a time by one wave (97 us: the others wait for it).
-constexpr int kSepTX = 64, kSepTY = 8;
 constexpr int kSepThreads = 64 * (kSepTY + 2);
 constexpr int kSepSide = 12;  // nine columns padded for 16-byte reads
-
-// Number of z chunks of the separable form for a grid, or 0 where the tiles
-// of stencil.h are faster.  Blocks beyond 256 share CUs, and a chunk of n
-// planes takes n + 2 plane steps, so the cost is (planes + 2) x ceil(blocks /
-// 256) steps of about 1.8 us (2.4 beyond the last-level cache); the 16x12x8
-// columns take about 32 us per 1024 blocks (both measured over 96x64x64 to
-// 384x256x256: 28 against 32 us at 160x96x96, 53 against 48 at 203x101x97).
-// Grids beyond the buffer accesses' 4 GiB take the tiles too.
-inline int sep3d_chunks(int nx, int ny, int nz, size_t plane) {
-  if ((10 * plane + (size_t)nx * ny) * sizeof(float) >= 0xFFFF0000ull) return 0;
-  const long long cols = (long long)((nx + kSepTX - 1) / kSepTX) * ((ny + kSepTY - 1) / kSepTY);
-  long long best = 0;
-  int chunks = 0;
-  for (int c = 1; c <= nz; c++) {
-    const long long blocks = cols * c, rounds = (blocks + 255) / 256;
-    const long long cost = ((nz + c - 1) / c + 2) * rounds;
-    if (!chunks || cost < best) {
-      best = cost;
-      chunks = c;
-    }
-  }
-  const long long tiles = (long long)((nx + 15) / 16) * ((ny + 11) / 12) * ((nz + 7) / 8);
-  return 57 * best < tiles ? chunks : 0;
-}
 
 // The domain's separable form: its z chunks, or 0 if it steps with the tiles.
 // A body or a wall keeps the tiles: their boundary cells and bounce-back work

@@ -19,8 +19,9 @@ __global__ void __launch_bounds__(kSepThreads, 5)
 }
 
 void plan3d(Domain& d) {
-  d.sep_chunks = sep3d_chunks(d.nx, d.ny, d.nz, d.plane);
-  d.row_chunks = rows3d_chunks(d.nx, d.ny, d.nz, d.plane, storage_planes(d.storage, 3), storage_bytes(d.storage));
+  const Grid3 g{d.nx, d.ny, d.nz};
+  d.sep_chunks = sep3d_chunks(g, d.plane);
+  d.row_chunks = rows3d_chunks(g, d.plane, storage_planes(d.storage, 3), storage_bytes(d.storage));
 }
 
 // The form of the domain's next step (FF_FORM_*) and the tile that it takes

@@ -1,0 +1,20 @@
+// Prints how 3D grids step (plan3d.h): for "nx ny nz" lines on the input, the
+// z chunks of the separable form and of whole rows (0: not that form) and the
+// default tile without and with a body, for FP32 and for 16-bit storage.
+#include <cstdio>
+
+#include "../../freeflow_amd/csrc/plan3d.h"
+
+int main() {
+  int nx, ny, nz;
+  while (std::scanf("%d %d %d", &nx, &ny, &nz) == 3) {
+    const ff::Grid3 g{nx, ny, nz};
+    const size_t plane = (size_t)(g.cells() + 255) / 256 * 256;
+    std::printf("%d", ff::sep3d_chunks(g, plane));
+    for (size_t elem : {4, 2})
+      std::printf(" %d %d %d", ff::rows3d_chunks(g, plane, 10, elem), ff::default_tile3(g, plane, 10, elem, false),
+                  ff::default_tile3(g, plane, 10, elem, true));
+    std::printf("\n");
+  }
+  return 0;
+}
