@@ -96,18 +96,28 @@ inline int rows3d_chunks(const Grid3& g, size_t plane, size_t planes, size_t ele
 //   104 / 90 against 66 / 56.  With a body the launch waits for its boundary
 //   cells too: 64^3 23.3 / 22.1 against 25.0 / 20.8, 96x64x64 30.4 / 27.8
 //   against 30.2 / 24.1, 160x96x96 84.7 / 73.6 against 56.1 / 45.0.
+//   Also where the columns are mostly padding: a box takes as long as 3.4
+//   plane steps of a column.  8x8x10000 33.4 / 26.9 against 45.5 / 34.8 (5.0
+//   steps a box), 8x100x1000 41.9 / 33.8 against 46.0 / 35.8 (3.46), but
+//   17x13x3500 65.9 / 51.8 against 59.1 / 46.2 (3.33).
 //   column 16x12x8 in between.
 //   column 32x12x16 once both moment buffers exceed the last-level cache, so
 //   that halo cells are read from memory again, and if its tiles are not
 //   padding for more than a fifth: 256x192x160 189 / 177 against 229 / 224
 //   (FP16 148 against 153), 384x256x256 650 / 622 against 811 / 807, but
 //   100x300x200 (33 % padding) 216 / 198 against 194 / 191, and FP16
-//   250x150x150 (225 MB) 126 against 103.
+//   250x150x150 (225 MB) 126 against 103; 1133x1837x2 147 against 174 (fast,
+//   one short column is no padding).  Also where the chunks of eight
+//   planes leave a remainder and one of sixteen does not: 196x850x11 51.0 /
+//   40.1 against 68.4 / 56.5, 293x378x9 42.8 / 33.5 against 50.2 / 41.9.
 inline int default_tile3(const Grid3& g, size_t plane, size_t planes, size_t elem, bool body) {
   const long long n = g.cells();
   if (n < (body ? 350000 : kColumnCells)) return 0;
-  const long long padded = g.tiles(32, 12) * 32 * 12 * ceil_div(g.nz, 16) * 16;
-  return beyond_cache(plane, planes, elem) && 5 * padded < 6 * n ? 15 : 7;
+  const long long boxes = g.tiles(8, 8) * ceil_div(g.nz, 4);
+  if ((double)(g.tiles(16, 12) * (g.nz + 2 * ceil_div(g.nz, 8))) > 3.4 * (double)boxes) return 0;
+  const long long padded = g.tiles(32, 12) * 32 * 12 * ceil_div(g.nz, 16) * std::min(g.nz, 16);
+  if (beyond_cache(plane, planes, elem)) return 5 * padded < 6 * n ? 15 : 7;
+  return columns15_us(g) < 0.9 * columns7_us(g) ? 15 : 7;
 }
 
 }  // namespace ff
