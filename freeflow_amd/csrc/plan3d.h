@@ -79,13 +79,19 @@ inline int sep3d_chunks(const Grid3& g, size_t plane) {
 // faster.  A step of 512 blocks takes as long as about 100 blocks of the
 // 16x12x8 column (2.6 us and 0.027 us a block in FP16 fast, 3.9 and 0.040 in
 // FP32 reference order): 51 us against 48 at 203x101x97, 33 against 31 at
-// 160x96x96 (padding to 64 cells), 69 against 75 at 256x128x128.  Buffers
-// beyond 4 GiB take the columns.
+// 160x96x96 (padding to 64 cells), 69 against 75 at 256x128x128.  Columns of
+// fewer than eight planes take n + 1 of 9 plane steps: FP32 reference order
+// 67.9 against 44.7 at 1000x1000x1, 50.8 / 44.4 at 690x429x5,
+// 910x352x2 33.2 / 25.7; level up to a ratio of 1.2 (66.0 / 61.6 at 800x700x4,
+// but FP16 19.9 / 20.6 at 122x1398x4).  Smaller grids would take boxes (22.0
+// against 29.3 at 692x233x3).  Buffers beyond 4 GiB take the columns.
 inline int rows3d_chunks(const Grid3& g, size_t plane, size_t planes, size_t elem) {
   if ((plane * planes + (size_t)g.nx * g.ny) * elem >= 0xFFFF0000ull) return 0;
   const RowChunks r = row_chunks(g.tiles(kRowsTX, kRowsTY), g.nz, 512);
   const long long blocks = g.tiles(16, 12) * ceil_div(g.nz, 8);
-  return 100 * r.steps < blocks ? r.chunks : 0;
+  if (100 * r.steps >= blocks) return 0;
+  if (g.cells() < kColumnCells) return r.chunks;
+  return 900.0 * (double)r.steps <= 1.2 * (double)((std::min(g.nz, 8) + 1) * blocks) ? r.chunks : 0;
 }
 
 // Tile of a domain whose tile was neither set nor tuned; any tile gives the

@@ -55,7 +55,7 @@ def plans(tmp_path_factory):
 
 def test_grids_on_both_sides_of_each_line(plans):
     for (g, sep, rows, tile, tile_body), p in zip(CASES, plans([c[0] for c in CASES])):
-        assert (p[0] > 0, p[2], p[3]) == (sep, tile, tile_body), (g, p)
+        assert (p[0] > 0, p[1] > 0, p[2], p[3]) == (sep, rows, tile, tile_body), (g, p)
 
 
 def test_chunks_lie_within_the_grid(plans):
