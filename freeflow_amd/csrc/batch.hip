@@ -159,7 +159,8 @@ template <int DIM, typename S, int FB>
 __global__ void __launch_bounds__(FB) kb_sums(const DomDev* __restrict__ doms, const int2* __restrict__ map) {
   const int2 m = map[blockIdx.x];
   const DomDev* D = doms + m.x;
-  elem_sums_body<DIM, S, FB, true>(D->la, D->fa, m.y, D->mom[(*D->step & 1u) ^ 1u]);
+  __shared__ SumsLds<DIM> lds;
+  elem_sums_body<DIM, S, FB, true>(D->la, D->fa, m.y, D->mom[(*D->step & 1u) ^ 1u], lds);
 }
 
 // Per domain: vertex blocks, then one block that folds the wrench, advances
@@ -286,7 +287,8 @@ template <int DIM>
 __global__ void __launch_bounds__(kSumBlock) kb_detect(const DomDev* __restrict__ doms, const int2* __restrict__ map) {
   const int2 m = map[blockIdx.x];
   const LinkArgs& la = doms[m.x].la;
-  detect_block<DIM, true>(la, (long long)m.y, step_tag(la), la.v[step_gen(la) & 1u]);
+  __shared__ DetLds<DIM> lds;
+  detect_block<DIM, true>(la, (long long)m.y, step_tag(la), la.v[step_gen(la) & 1u], lds);
 }
 
 // Block size of the stream launch for a tile index.
@@ -402,10 +404,10 @@ static int build_tables(Batch& b, int tile) {
       r.ndet = detect_blocks(d, true);
       r.fa.copy_blocks = copyback_blocks(d, kSumBlock, 4);  // fewer blocks: many domains share the launch
     } else {
-      r.la.ne = 0;
+      r.la.ne = r.la.neb = 0;
       r.fa.copy_blocks = 0;
     }
-    const int nes = (bnd ? elem_blocks(b.dim, d.ne) : 0) + r.fa.outlet_blocks + r.fa.copy_blocks + r.ndet;
+    const int nes = r.la.neb + r.fa.outlet_blocks + r.fa.copy_blocks + r.ndet;
     for (int t = 0; t < nes; t++) es.push_back(make_int2(i, t));
     for (int t = 0; t <= r.nvb; t++) fin.push_back(make_int2(i, t));
   }

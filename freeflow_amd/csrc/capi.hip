@@ -392,6 +392,8 @@ LinkArgs link_args(Domain& d, const float* v0, const float* v1, const float* u0,
   la.sb = d.lk_sb;
   la.cap = d.lt_cap;
   la.bc_span = bc_span(d);
+  la.epb = d.epb;
+  la.neb = (d.ne + d.epb - 1) / d.epb;
   la.st = d.st;
   la.gen = d.gen_host;
   la.tag = d.tag_host;
@@ -711,6 +713,7 @@ int ff_set_boundary(ff_domain* dd, int nv, const float* verts, const float* vels
       if (cnt[b]) for (int c = 0; c < D; c++) ref[(size_t)b * D + c] /= cnt[b];
     for (int v = 0; v < nv; v++) if (vb[v] < 0) vb[v] = 0;
   }
+  d.epb = elements_per_block(d, verts, elems);
   // link table capacity: distinct candidate cells near the mesh, with margin
   const unsigned long long est = link_estimate(D, d.dx, ne, verts, elems);
   d.lt_cap = (int)next_pow2(est * 2 + 1024);

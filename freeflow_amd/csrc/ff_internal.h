@@ -73,6 +73,7 @@ struct LinkArgs {
   float* lh;                  // cap * (Q-1) * DIM  hit point
   float* sb;                  // cap * NM  updated moments of each boundary cell (copied back after the step)
   int cap;
+  int epb, neb;  // elements in a block of the element sums (and of the 3D detection), blocks
   int bc_span;  // link-table slots a boundary-cell block scans per pass (<= its block size)
   StepState* st;
   // Step generation (vertex-buffer parity gen & 1, wrench ring slot) and
@@ -114,6 +115,7 @@ struct Domain {
   int n_outlets = 0;
   // boundary geometry (device, interleaved like the reference proxy)
   int nv = 0, ne = 0, n_bodies = 0;
+  int epb = 1;  // elements in a block of the element sums (LinkArgs)
   void* bnd_mem = nullptr;   // one allocation holding the ff_set_boundary arrays below
   void* core_mem = nullptr;  // one allocation holding the moments, flags and reduction scratch
   float* vbuf[2] = {nullptr, nullptr};  // positions by generation parity
@@ -244,6 +246,7 @@ int launch_wave_now(Domain& d);
 // and 8 FP32 values derived from them for the fast-math kinematics.
 constexpr int kWaveParStride = 8;  // doubles per body
 void wave_device_params(const double* p4, double dt, int n_bodies, double* out);
+int elements_per_block(const Domain& d, const float* verts, const uint32_t* elems);
 int detect_blocks(const Domain& d, bool batched);  // detection blocks of 256 threads
 int bc_span(const Domain& d);  // boundary-cell scan span of a domain stepped on its own
 int launch_step_vertex_forces(Domain& d, float* out_dev);

@@ -418,9 +418,6 @@ __device__ __forceinline__ void build_links_pairs2(const LinkArgs& la, long long
   }
 }
 
-// Capacity of build_links_block3's LDS lists.
-constexpr int kDet3Cap = 4096;
-
 // Superset test, without a division, of "num / den rounds into [0, 1] or is
 // NaN" (the plane-parameter test of line_triangle_intersect): num = 0 gives
 // +-0 or NaN; a zero den otherwise gives +-inf; equal signs need
@@ -434,39 +431,60 @@ __device__ __forceinline__ bool tri3_t_may_pass(float num, float den) {
   return (num > 0.0f) == (den > 0.0f) ? an <= ad * 1.0001f : an < ad * 1e-30f;
 }
 
-// 3D link detection with one 256-thread block per element, cell-major: each
-// thread takes two cells of the element's window per pass, forms
-// num = n . (v0 - p1), and only cells within 2 cl of the triangle's plane go
-// on (no link of length <= sqrt(3) cl from a farther cell reaches it; the
-// margin is far above the rounding of the link ends for grids up to millions
-// of cells per axis).  Their 26 links (unrolled, lattice vectors as constants)
-// whose plane parameter t = num / (n . dd) may lie in [0, 1] (tri3_t_may_pass,
-// no division) form a bit mask; a block-wide prefix sum of the masks' counts
-// lists the survivors in LDS, all threads finish them (t itself, parallel
-// test, barycentrics), and the hits, listed again, are entered in the table
-// together.  Bound by the chain of loads, barriers and table round trips of
-// one block: one list position per direction from an LDS counter, with a
-// barrier every fourth, took 21 us for the 320 triangles of a sphere.
-__device__ __forceinline__ void build_links_block3(const LinkArgs& la, long long block, unsigned tag, const float* v) {
-  constexpr int K = 26, NT = 256, NW = NT / 64, U = 2;
-  __shared__ int s_wave[NW], s_nhit;
-  __shared__ unsigned short s_may[kDet3Cap], s_hit[kDet3Cap];
-  if (block >= (long long)la.ne) return;  // block-uniform
-  const int elem = (int)block;
+// Threads that handle one triangle in the 3D detection and element sums: a
+// block, or a wave (la.epb = 4) where the elements fill the chip anyway.
+constexpr int kBlock3 = 256;
+template <int NT>
+__device__ __forceinline__ void group_sync() {
+  if constexpr (NT == 64) {  // one wave: its LDS accesses are in order, the compiler's need to be
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  } else {
+    __syncthreads();
+  }
+}
+
+// Lists of links of build_links_group3.
+template <int NT>
+struct Det3Lists {
+  static constexpr int CAP = 16 * NT;
+  unsigned short may[CAP], hit[CAP];
+  int wave[NT / 64], nhit;
+};
+
+// 3D link detection with NT threads per element, cell-major: each thread takes
+// U cells of the element's window per pass, forms num = n . (v0 - p1), and only
+// cells within 2 cl of the triangle's plane go on (no link of length <= sqrt(3)
+// cl from a farther cell reaches it; the margin is far above the rounding of
+// the link ends for grids up to millions of cells per axis).  Their 26 links
+// (unrolled, lattice vectors as constants) whose plane parameter t = num / (n .
+// dd) may lie in [0, 1] (tri3_t_may_pass, no division) form a bit mask; a
+// prefix sum of the masks' counts lists the survivors in LDS, all threads
+// finish them (t itself, parallel test, barycentrics), and the hits, listed
+// again, are entered in the table together.  A block per element is bound by
+// its chain of loads, barriers and table round trips: one list position per
+// direction from an LDS counter, with a barrier every fourth, took 21 us for
+// the 320 triangles of a sphere.
+template <int NT>
+__device__ __forceinline__ void build_links_group3(const LinkArgs& la, int elem, unsigned tag, const float* v,
+                                                   Det3Lists<NT>& lds) {
+  constexpr int K = 26, NW = NT / 64, U = NT == 64 ? 1 : 2, CAP = Det3Lists<NT>::CAP;
+  static_assert(U * NT <= 2048, "a cell of the pass and a direction in 16 bits");
   const int n[3] = {la.nx, la.ny, la.nz};
   const uint32_t* e = dev_global(la.e);
   v = dev_global(v);
   int lo[3], hi[3];
   elem_window<3>(v, e, elem, la.cl, n, lo, hi);
   const int wx = hi[0] - lo[0] + 1, wy = hi[1] - lo[1] + 1, wz = hi[2] - lo[2] + 1;
-  if (wx <= 0 || wy <= 0 || wz <= 0) return;  // block-uniform
+  if (wx <= 0 || wy <= 0 || wz <= 0) return;  // the same for the whole group, as every branch around a group_sync
   const int ncell = wx * wy * wz;
   const Tri3 T = tri3(v, e, elem);
   const float far = 2.0f * la.cl;
   const uint8_t* flags = dev_global(la.flags);
   unsigned long long* cells = table_cells(la, tag);
   unsigned long long* keys = table_keys<3>(la, tag);
-  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = (int)threadIdx.x & (NT - 1), lane = tid & 63, wave = tid >> 6;
   // link q of the pass at c0: bits 5.. the cell's place in the pass, 0-4 the direction
   auto link_test = [&](int c0, unsigned q, int& cell, int& l, Hit& h) {
     const int k = c0 + (int)(q >> 5);
@@ -483,7 +501,7 @@ __device__ __forceinline__ void build_links_block3(const LinkArgs& la, long long
     unsigned may[U];
     bool upd[U];
 #pragma unroll
-    for (int w = 0; w < U; w++) {  // both flags in flight
+    for (int w = 0; w < U; w++) {  // the flags in flight together
       const int k = c0 + w * NT + tid;
       upd[w] = false;
       if (k < ncell) {
@@ -513,70 +531,93 @@ __device__ __forceinline__ void build_links_block3(const LinkArgs& la, long long
       }
       count += __popc(may[w]);
     }
-    // block-wide prefix sum of the counts
+    // prefix sum of the counts over the group
     int before = count;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
       const int o = __shfl_up(before, off, 64);
       if (lane >= off) before += o;
     }
-    if (lane == 63) s_wave[wave] = before;
-    __syncthreads();
-    before -= count;
     int total = 0;
+    if constexpr (NW == 1) {
+      total = __shfl(before, 63, 64);
+      before -= count;
+    } else {
+      if (lane == 63) lds.wave[wave] = before;
+      group_sync<NT>();
+      before -= count;
 #pragma unroll
-    for (int w = 0; w < NW; w++) {
-      before += w < wave ? s_wave[w] : 0;
-      total += s_wave[w];
+      for (int w = 0; w < NW; w++) {
+        before += w < wave ? lds.wave[w] : 0;
+        total += lds.wave[w];
+      }
     }
-    for (int base = 0; base < total; base += kDet3Cap) {
-      if (tid == 0) s_nhit = 0;
+    for (int base = 0; base < total; base += CAP) {
+      if (tid == 0) lds.nhit = 0;
       int at = before - base;
 #pragma unroll
       for (int w = 0; w < U; w++)
         for (unsigned m = may[w]; m; m &= m - 1, at++)
-          if (at >= 0 && at < kDet3Cap)
-            s_may[at] = (unsigned short)(((w * NT + tid) << 5) | (__ffs((int)m) - 1));
-      __syncthreads();
-      const int ns = min(total - base, kDet3Cap);
+          if (at >= 0 && at < CAP) lds.may[at] = (unsigned short)(((w * NT + tid) << 5) | (__ffs((int)m) - 1));
+      group_sync<NT>();
+      const int ns = min(total - base, CAP);
       for (int q0 = 0; q0 < ns; q0 += NT) {
         const int q = q0 + tid;
         int cell, l;
         Hit h;
-        const bool hit = q < ns && link_test(c0, s_may[q], cell, l, h);
+        const bool hit = q < ns && link_test(c0, lds.may[q], cell, l, h);
         const unsigned long long m = __ballot(hit);
         if (m) {
           int pos = 0;
-          if (lane == 0) pos = atomicAdd(&s_nhit, (int)__popcll(m));
+          if (lane == 0) pos = atomicAdd(&lds.nhit, (int)__popcll(m));
           pos = __shfl(pos, 0, 64);
-          if (hit) s_hit[pos + (int)__popcll(m & ((1ull << lane) - 1ull))] = s_may[q];
+          if (hit) lds.hit[pos + (int)__popcll(m & ((1ull << lane) - 1ull))] = lds.may[q];
         }
       }
-      __syncthreads();
-      const int nh = s_nhit;
+      group_sync<NT>();
+      const int nh = lds.nhit;
       for (int q = tid; q < nh; q += NT) {
         int cell, l;
         Hit h;
-        link_test(c0, s_hit[q], cell, l, h);
+        link_test(c0, lds.hit[q], cell, l, h);
         const int slot = lt_claim(cells, la.cap, tag, cell, &la.st->overflow);
         if (slot >= 0) lt_offer_key(keys, (size_t)slot * K + (l - 1), tag, depth_key(h.depth, elem));
       }
-      __syncthreads();  // the lists and counters are free again
+      group_sync<NT>();  // the lists and counters are free again
     }
-    if (total == 0) __syncthreads();  // s_wave is read before the next pass writes it
+    if (total == 0) group_sync<NT>();  // lds.wave is read before the next pass writes it
   }
 }
 
+// LDS of a detection block.
+template <int DIM>
+struct DetLds {};
+template <>
+struct DetLds<3> {
+  union {
+    Det3Lists<kBlock3> block;
+    Det3Lists<64> wave[kBlock3 / 64];
+  };
+};
+
 // Detection block of 256 threads: 2D takes blockDim / kRow elements (ROWS) or
-// (element, direction) pairs, 3D one element.
+// (element, direction) pairs, 3D la.epb elements.
 template <int DIM, bool ROWS>
-__device__ __forceinline__ void detect_block(const LinkArgs& la, long long block, unsigned tag, const float* v) {
-  if constexpr (DIM == 3)
-    build_links_block3(la, block, tag, v);
-  else if constexpr (ROWS)
+__device__ __forceinline__ void detect_block(const LinkArgs& la, long long block, unsigned tag, const float* v,
+                                             DetLds<DIM>& lds) {
+  if constexpr (DIM == 3) {
+    if (la.epb == 1) {
+      if (block < la.ne) build_links_group3<kBlock3>(la, (int)block, tag, v, lds.block);
+    } else {
+      const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+      const long long elem = block * (kBlock3 / 64) + wave;
+      if (elem < la.ne) build_links_group3<64>(la, (int)elem, tag, v, lds.wave[wave]);
+    }
+  } else if constexpr (ROWS) {
     build_links_rows2(la, block, tag, v);
-  else
+  } else {
     build_links_pairs2(la, block, tag, v);
+  }
 }
 
 }  // namespace ff

@@ -46,7 +46,8 @@ namespace ff {
 // Links of the current step under the current tag and vertex buffer.
 template <int DIM>
 __global__ void __launch_bounds__(256) k_links_build(LinkArgs la) {
-  detect_block<DIM, false>(la, blockIdx.x, step_tag(la), la.v[step_gen(la) & 1]);
+  __shared__ DetLds<DIM> lds;
+  detect_block<DIM, false>(la, blockIdx.x, step_tag(la), la.v[step_gen(la) & 1], lds);
 }
 
 // Links of the current step of a domain stepped on its own (a batch detects
@@ -65,7 +66,8 @@ int launch_detect(Domain& d, const LinkArgs& la) {
 // Element sums, outlets, copy-back and next-step detection.
 template <int DIM, typename S, int FB>
 __global__ void __launch_bounds__(FB) k_step_sums(LinkArgs la, FinalArgs fa, void* out) {
-  elem_sums_body<DIM, S, FB, false>(la, fa, blockIdx.x, out);
+  __shared__ SumsLds<DIM> lds;
+  elem_sums_body<DIM, S, FB, false>(la, fa, blockIdx.x, out, lds);
 }
 
 // Vertex blocks, then one last block for the body wrenches and the advance
@@ -80,9 +82,43 @@ __global__ void __launch_bounds__(FB) k_step_finish(LinkArgs la, FinalArgs fa, i
   else finish_last_body<DIM, FB>(la, fa, fa.fin_gen, false, lds);
 }
 
+// Elements in a block of the sums launch and of the 3D detection.
+// 2D: kRow lanes each.  3D: a block each where the launch waits for its slowest
+// block, a wave each (the same bits) where many triangles with windows of few
+// cells would leave most of a block's threads without one.  us a step, block
+// / wave, of a body at rest in 160x96x96 (in brackets eight of them as a
+// batch); mean window in cells:
+//     320 triangles, 206 cells   64 /  92 [ 513 /  519]
+//    1280 triangles,  90 cells   82 /  71 [ 677 /  556]
+//    1280 triangles, 262 cells  172 / 176 [1241 / 1202]
+//    5120 triangles,  53 cells  139 /  90 [1176 /  710]
+//   20480 triangles,  57 cells  502 / 288 [4087 / 2100]
+//      12 triangles, thousands  266 / 791 [ 708 / 1430]
+int elements_per_block(const Domain& d, const float* verts, const uint32_t* elems) {
+  if (d.dim == 2) return kSumBlock / kRow;
+  if (d.ne <= 512) return 1;
+  const int n[3] = {d.nx, d.ny, d.nz};
+  double cells = 0.0;  // of the candidate windows (elem_window)
+  for (int k = 0; k < d.ne; k++) {
+    double w = 1.0;
+    for (int c = 0; c < 3; c++) {
+      double mn = 1e300, mx = 0.0;
+      for (int j = 0; j < 3; j++) {
+        const double x = verts[(size_t)elems[(size_t)k * 3 + j] * 3 + c] / d.dx;
+        mn = std::min(mn, x);
+        mx = std::max(mx, x);
+      }
+      const double lo = std::max(std::trunc(mn) - 1.0, 0.0), hi = std::min(std::trunc(mx) + 1.0, n[c] - 1.0);
+      w *= std::max(hi - lo + 1.0, 0.0);
+    }
+    cells += w;
+  }
+  return cells <= 128.0 * d.ne ? kSumBlock / 64 : 1;
+}
+
 // Detection blocks of 256 threads (detect_block).
 int detect_blocks(const Domain& d, bool batched) {
-  if (d.dim == 3) return d.ne;
+  if (d.dim == 3) return (d.ne + d.epb - 1) / d.epb;
   constexpr int per = 256 / kRow;
   const int n = batched ? d.ne : d.ne * (d.q - 1);  // at most 65536 elements
   return (n + per - 1) / per;
@@ -116,7 +152,7 @@ int launch_step_sums(Domain& d, const LinkArgs& la, void* out, bool detect_next)
   constexpr int FB = kSumBlock;
   const FinalArgs fa = make_final_args(d, out, d.vbuf[0], d.vbuf[1], d.ubuf[0], d.ubuf[1], nullptr);
   const unsigned grid =
-      (unsigned)(elem_blocks(d.dim, d.ne) + fa.outlet_blocks + fa.copy_blocks + (detect_next ? detect_blocks(d, false) : 0));
+      (unsigned)(la.neb + fa.outlet_blocks + fa.copy_blocks + (detect_next ? detect_blocks(d, false) : 0));
 #define FF_SUM(DIM, S) k_step_sums<DIM, S, FB><<<grid, FB, 0, d.stream>>>(la, fa, out)
   if (d.dim == 2) {
     if (d.storage == FF_STORAGE_F32) FF_SUM(2, float);

@@ -266,14 +266,9 @@ struct FinalArgs {
   unsigned fin_gen;
 };
 
-// Block size of the element-sum launch, and blocks for the sums of `ne`
-// elements: kRow lanes per segment in 2D, a block per triangle in 3D (see
-// elem_sum2 / elem_sum3).
+// Block size of the element-sum launch (elements_per_block).
 constexpr int kSumBlock = 256;
-__host__ __device__ inline int elem_blocks(int dim, int ne) {
-  constexpr int per = kSumBlock / kRow;
-  return dim == 2 ? (ne + per - 1) / per : ne;
-}
+static_assert(kSumBlock == kBlock3, "a block of the element sums and of the detection takes the same triangles");
 
 // Host: the FinalArgs of a domain (outlets written into `out`, next-step
 // kinematics into vn/un, per-vertex forces optionally added to proxy_forces).
@@ -351,9 +346,9 @@ __device__ __forceinline__ void wave_block_body(const LinkArgs& la, const FinalA
 // Detection of the next step's links (tag + 1, the next step's vertex
 // positions) into the other link table.
 template <int DIM, bool BATCHED>
-__device__ __forceinline__ void detect_next_body(const LinkArgs& la, int blk) {
+__device__ __forceinline__ void detect_next_body(const LinkArgs& la, int blk, DetLds<DIM>& lds) {
   const unsigned gen = step_gen(la);
-  detect_block<DIM, BATCHED>(la, (long long)blk, step_tag(la) + 1u, la.v[(gen + 1u) & 1u]);
+  detect_block<DIM, BATCHED>(la, (long long)blk, step_tag(la) + 1u, la.v[(gen + 1u) & 1u], lds);
 }
 
 // ---------------------------------------------------------------- element sums
@@ -493,16 +488,20 @@ __device__ __forceinline__ void elem_sum2(const LinkArgs& la, const FinalArgs& f
   }
 }
 
-// Sum of one triangle's links by a block of kSumBlock threads: a window of
-// some 7^3 cells, one cell per thread and pass, its 26 keys read as one row.
-// One wave per triangle walked the same window in six passes of (cell,
-// direction) tasks, a serial chain of some 150 loads that set the launch's
-// time (76 us for the 320 triangles of a sphere in a 160x96x96 domain).
-// The rows of 16 lanes are folded by a fixed tree, their sums in row order.
-__device__ __forceinline__ void elem_sum3(const LinkArgs& la, const FinalArgs& fa, int elem) {
-  constexpr int K = 26, STRIDE = elem_stride_v<3>, M = STRIDE - 1, NROW = kSumBlock / kRow;
+// Sum of one triangle's links by NT threads: a window of some 4^3 to 7^3
+// cells, one cell per thread and pass, its 26 keys read as one row.  The cells
+// belong to the kBlock3 threads of a block in turn, whose rows of 16 are folded
+// by a fixed tree and their sums in row order; a wave (NT = 64) takes the
+// block's four waves one after the other, so the sums are the same bits.
+// One wave per triangle with (cell, direction) tasks walked the window of a
+// triangle of a sphere of 320 in a serial chain of some 150 loads, which set
+// the launch's time (76 us in a 160x96x96 domain).
+using Sum3Part = double[kBlock3 / kRow][kRow];
+template <int NT>
+__device__ __forceinline__ void elem_sum3(const LinkArgs& la, const FinalArgs& fa, int elem, Sum3Part& part) {
+  constexpr int K = 26, STRIDE = elem_stride_v<3>, M = STRIDE - 1, NROW = kBlock3 / kRow;
   static_assert(M <= kRow, "one lane of a row per sum");
-  __shared__ double s_part[NROW][kRow];
+  const int tid = (int)threadIdx.x & (NT - 1);
   const unsigned gen = step_gen(la), tag = step_tag(la);
   const float* v = dev_global(la.v[gen & 1]);
   const int n[3] = {la.nx, la.ny, la.nz};
@@ -514,9 +513,6 @@ __device__ __forceinline__ void elem_sum3(const LinkArgs& la, const FinalArgs& f
   double ref[3];
 #pragma unroll
   for (int c = 0; c < 3; c++) ref[c] = dev_global(fa.body_ref)[body * 3 + c];
-  double acc[M];
-#pragma unroll
-  for (int a = 0; a < M; a++) acc[a] = 0.0;
   const unsigned etag = (unsigned)elem & 0xFFFFu;
   const uint8_t* flags = dev_global(la.flags);
   const unsigned long long* cells = table_cells(la, tag);
@@ -524,51 +520,57 @@ __device__ __forceinline__ void elem_sum3(const LinkArgs& la, const FinalArgs& f
   const float* lf = dev_global(la.lf);
   const float* lb = dev_global(la.lb);
   const float* lh = dev_global(la.lh);
-  for (int k = (int)threadIdx.x; k < ncell; k += kSumBlock) {
-    const int i = lo[0] + k % wx, j = lo[1] + (k / wx) % wy, z = lo[2] + k / (wx * wy);
-    const int cell = (z * la.ny + j) * la.nx + i;
-    const unsigned home = lt_home(la.cap, cell);
-    const unsigned long long cur = cells[home];
-    if (!is_updated(flags[cell])) continue;
-    const int slot = lt_resolve(cells, la.cap, tag, cell, home, cur);
-    if (slot < 0) continue;
-    for (unsigned m = links_of_element<3>(keys, slot, tag, etag); m; m &= m - 1) {
-      const size_t li = ((size_t)slot * K + (__ffs((int)m) - 1)) * 3;
-      float F[3], B[3], H[3];
+  const int lane = tid % kRow, nq = min(kBlock3 / NT, max(1, (ncell + NT - 1) / NT));
+  for (int q = 0; q < nq; q++) {
+    double acc[M];
 #pragma unroll
-      for (int c = 0; c < 3; c++) {
-        F[c] = lf[li + c];
-        B[c] = lb[li + c];
-        H[c] = lh[li + c];
+    for (int a = 0; a < M; a++) acc[a] = 0.0;
+    for (int k = q * NT + tid; k < ncell; k += kBlock3) {
+      const int i = lo[0] + k % wx, j = lo[1] + (k / wx) % wy, z = lo[2] + k / (wx * wy);
+      const int cell = (z * la.ny + j) * la.nx + i;
+      const unsigned home = lt_home(la.cap, cell);
+      const unsigned long long cur = cells[home];
+      if (!is_updated(flags[cell])) continue;
+      const int slot = lt_resolve(cells, la.cap, tag, cell, home, cur);
+      if (slot < 0) continue;
+      for (unsigned m = links_of_element<3>(keys, slot, tag, etag); m; m &= m - 1) {
+        const size_t li = ((size_t)slot * K + (__ffs((int)m) - 1)) * 3;
+        float F[3], B[3], H[3];
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          F[c] = lf[li + c];
+          B[c] = lb[li + c];
+          H[c] = lh[li + c];
+        }
+        if (B[0] == kLinkUnused) continue;
+#pragma unroll
+        for (int jv = 0; jv < 3; jv++)
+#pragma unroll
+          for (int c = 0; c < 3; c++) acc[jv * 3 + c] += (double)(F[c] * B[jv]);  // addForceAt products
+        double r[3];
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          acc[9 + c] += (double)F[c];
+          r[c] = (double)H[c] - ref[c];
+        }
+        acc[12] += r[1] * (double)F[2] - r[2] * (double)F[1];
+        acc[13] += r[2] * (double)F[0] - r[0] * (double)F[2];
+        acc[14] += r[0] * (double)F[1] - r[1] * (double)F[0];
       }
-      if (B[0] == kLinkUnused) continue;
+    }
+    row_sums<M>(acc);
+    if (lane == 0) {
 #pragma unroll
-      for (int jv = 0; jv < 3; jv++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) acc[jv * 3 + c] += (double)(F[c] * B[jv]);  // addForceAt products
-      double r[3];
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        acc[9 + c] += (double)F[c];
-        r[c] = (double)H[c] - ref[c];
-      }
-      acc[12] += r[1] * (double)F[2] - r[2] * (double)F[1];
-      acc[13] += r[2] * (double)F[0] - r[0] * (double)F[2];
-      acc[14] += r[0] * (double)F[1] - r[1] * (double)F[0];
+      for (int a = 0; a < M; a++) part[(q * NT + tid) / kRow][a] = acc[a];
     }
   }
-  row_sums<M>(acc);
-  const int row = (int)threadIdx.x / kRow, lane = (int)threadIdx.x % kRow;
-  if (lane == 0) {
-#pragma unroll
-    for (int a = 0; a < M; a++) s_part[row][a] = acc[a];
-  }
-  __syncthreads();
-  if ((int)threadIdx.x < kRow) {
+  group_sync<NT>();
+  if (tid < kRow) {
     double t = 0.0;
     if (lane < M) {
 #pragma unroll
-      for (int r = 0; r < NROW; r++) t += s_part[r][lane];
+      for (int r = 0; r < NROW; r++)
+        if (NT == kBlock3 || r < nq * (NT / kRow)) t += part[r][lane];  // the other rows have no cell: zero
     }
     // the element's power: its vertex shares against the velocities the step used
     double pw = 0.0;
@@ -583,6 +585,17 @@ __device__ __forceinline__ void elem_sum3(const LinkArgs& la, const FinalArgs& f
   }
 }
 
+// LDS of a block of the element-sum launch.
+template <int DIM>
+union SumsLds {
+  DetLds<DIM> det;
+  Sum3Part part[kBlock3 / 64];
+};
+template <>
+union SumsLds<2> {
+  DetLds<2> det;
+};
+
 // Second launch of a boundary step, kSumBlock threads per block.  The first
 // elem_blocks blocks sum links per element (fixed order, FP64) into elem_acc.
 // Then outlet blocks: outlet cells of the freshly written buffer
@@ -591,12 +604,13 @@ __device__ __forceinline__ void elem_sum3(const LinkArgs& la, const FinalArgs& f
 // launch writes).  Then copy-back blocks: boundary-cell rows into the output.
 // Any further blocks detect the next step's links.
 template <int DIM, typename S, int FB, bool BATCHED>
-__device__ __forceinline__ void elem_sums_body(const LinkArgs& la, const FinalArgs& fa, int blk, void* out) {
+__device__ __forceinline__ void elem_sums_body(const LinkArgs& la, const FinalArgs& fa, int blk, void* out,
+                                               SumsLds<DIM>& lds) {
   static_assert(FB == kSumBlock, "element sums and detection are written for kSumBlock threads");
   constexpr int NM = DIM == 2 ? 6 : 10;
-  const int neb = elem_blocks(DIM, la.ne);
+  const int neb = la.neb;
   if (blk >= neb + fa.outlet_blocks + fa.copy_blocks) {
-    detect_next_body<DIM, BATCHED>(la, blk - neb - fa.outlet_blocks - fa.copy_blocks);
+    detect_next_body<DIM, BATCHED>(la, blk - neb - fa.outlet_blocks - fa.copy_blocks, lds.det);
     return;
   }
   if (blk >= neb + fa.outlet_blocks) {
@@ -640,8 +654,12 @@ __device__ __forceinline__ void elem_sums_body(const LinkArgs& la, const FinalAr
   if constexpr (DIM == 2) {
     const int elem = blk * (FB / kRow) + (int)threadIdx.x / kRow;
     if (elem < la.ne) elem_sum2(la, fa, elem, (int)threadIdx.x % kRow);
+  } else if (la.epb == 1) {
+    elem_sum3<kBlock3>(la, fa, blk, lds.part[0]);
   } else {
-    elem_sum3(la, fa, blk);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int elem = blk * (FB / 64) + wave;
+    if (elem < la.ne) elem_sum3<64>(la, fa, elem, lds.part[wave]);
   }
 }
 

@@ -1,0 +1,55 @@
+"""3D element sums and link detection by a wave per triangle, which meshes of
+many small triangles take in place of a block per triangle: against the oracle
+(bounds as in test_gpu_boundary_edges), element counts that are no multiple of
+the four waves of a block, windows of one pass of a wave to many and lists that
+overflow; and the same bits as the block form, alone and in a batch."""
+import numpy as np
+import pytest
+
+from freeflow_amd import capi, workloads as wl
+from test_gpu_boundary_edges import run_pair
+
+pytestmark = pytest.mark.gpu
+
+
+def bodies(*parts):
+    """One mesh of several (vertices, elements); returns it with the body of each element."""
+    v = np.concatenate([p[0] for p in parts])
+    off = np.cumsum([0] + [len(p[0]) for p in parts])
+    e = np.concatenate([p[1] + o for p, o in zip(parts, off)]).astype(np.uint32)
+    return v, e, np.repeat(np.arange(len(parts)), [len(p[1]) for p in parts]).astype(np.int32)
+
+
+@pytest.mark.parametrize("drop,big", [(0, None), (1, None), (2, None), (3, 13.0), (0, 9.0)])
+def test_fine_meshes(drop, big):
+    print(f"case fine mesh drop={drop} big={big}", flush=True)
+    v, e = wl.icosphere([17.3, 16.2, 15.6], 6.5 if big is None else 3.7, 3)
+    e = e[:len(e) - drop]
+    if big is not None:  # 20 triangles whose windows hold hundreds to thousands of cells
+        v, e, _ = bodies((v, e), wl.icosphere([18.1, 16.4, 15.2], big, 0))
+    vel = np.tile([0.02, -0.01, 0.015], (len(v), 1))
+    a = run_pair(3, (36, 33, 32), v, vel, e, 2, False)
+    b = run_pair(3, (36, 33, 32), v, vel, e, 2, True)
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
+def test_wave_and_block_give_the_same_sums():
+    """A body of 20 triangles alone (blocks) and beside a fine one far away
+    (waves): its first step is the same."""
+    grid = (72, 33, 32)
+    print(f"case wave against block {grid}", flush=True)
+    big, fine = wl.icosphere([17.3, 16.2, 15.6], 8.2, 0), wl.icosphere([55.1, 16.2, 15.4], 4.1, 3)
+    m = wl.equilibrium_moments(np.random.default_rng(3).uniform(-0.02, 0.02, (72 * 33 * 32, 3))).astype(np.float32)
+    out = []
+    for parts in ((big,), (big, fine)):
+        d = capi.Domain(3, *grid, viscosity=0.02)
+        d.set_moments(m)
+        v, e, b = bodies(*parts)
+        d.set_boundary(v, np.tile([0.02, -0.01, 0.015], (len(v), 1)), e, b, len(parts))
+        d.set_body_ref(np.tile([17.0, 16.0, 15.0], (len(parts), 1)))
+        d.step(1)
+        out.append((d.body_wrench()[0], d.body_power()[0], d.step_vertex_forces()[:len(big[0])]))
+        d.close()
+    assert np.abs(out[0][0]).min() > 0
+    for x, y in zip(*out):
+        assert np.array_equal(x, y)
