@@ -82,29 +82,38 @@ __global__ void __launch_bounds__(FB) k_step_finish(LinkArgs la, FinalArgs fa, i
   else finish_last_body<DIM, FB>(la, fa, fa.fin_gen, false, lds);
 }
 
-// Elements in a block of the sums launch and of the 3D detection.
-// 2D: kRow lanes each.  3D: a block each where the launch waits for its slowest
-// block, a wave each (the same bits) where many triangles with windows of few
-// cells would leave most of a block's threads without one.  us a step, block
-// / wave, of a body at rest in 160x96x96 (in brackets eight of them as a
-// batch); mean window in cells:
+// Elements in a block of the sums launch and of the 3D detection, by their
+// candidate windows.  us a step of a body at rest, in brackets of many as a
+// batch (eight in 3D, 32 in 2D).
+// 3D: a block each where the launch waits for its slowest block, a wave each
+// (the same bits) where many triangles with windows of few cells would leave
+// most of a block's threads without one.  160x96x96, block / wave, with the
+// mean window:
 //     320 triangles, 206 cells   64 /  92 [ 513 /  519]
 //    1280 triangles,  90 cells   82 /  71 [ 677 /  556]
 //    1280 triangles, 262 cells  172 / 176 [1241 / 1202]
 //    5120 triangles,  53 cells  139 /  90 [1176 /  710]
 //   20480 triangles,  57 cells  502 / 288 [4087 / 2100]
 //      12 triangles, thousands  266 / 791 [ 708 / 1430]
+// 2D: kRow lanes each, or a block each where the launch would wait for one
+// long segment; the same choice alone and in a batch, whose sums are the same
+// bits.  1000x400, kRow lanes / block, with the largest window:
+//       4 segments, 6716 cells  359 / 305 [ 949 /  928]
+//      12 segments,  980 cells   97 /  79 [ 426 /  441]
+//      24 segments,  306 cells   46 /  41 [ 277 /  288]
+//      48 segments,  110 cells   24 /  23 [ 236 /  246]
+//     600 segments,   16 cells   17 /  18 [ 230 /  292]
+//    4000 segments,    9 cells   23 /  31 [ 289 /  638]
 int elements_per_block(const Domain& d, const float* verts, const uint32_t* elems) {
-  if (d.dim == 2) return kSumBlock / kRow;
-  if (d.ne <= 512) return 1;
+  if (d.dim == 3 && d.ne <= 512) return 1;
   const int n[3] = {d.nx, d.ny, d.nz};
-  double cells = 0.0;  // of the candidate windows (elem_window)
+  double cells = 0.0, largest = 0.0;  // of the windows (elem_window)
   for (int k = 0; k < d.ne; k++) {
     double w = 1.0;
-    for (int c = 0; c < 3; c++) {
+    for (int c = 0; c < d.dim; c++) {
       double mn = 1e300, mx = 0.0;
-      for (int j = 0; j < 3; j++) {
-        const double x = verts[(size_t)elems[(size_t)k * 3 + j] * 3 + c] / d.dx;
+      for (int j = 0; j < d.dim; j++) {
+        const double x = verts[(size_t)elems[(size_t)k * d.dim + j] * d.dim + c] / d.dx;
         mn = std::min(mn, x);
         mx = std::max(mx, x);
       }
@@ -112,8 +121,10 @@ int elements_per_block(const Domain& d, const float* verts, const uint32_t* elem
       w *= std::max(hi - lo + 1.0, 0.0);
     }
     cells += w;
+    largest = std::max(largest, w);
   }
-  return cells <= 128.0 * d.ne ? kSumBlock / 64 : 1;
+  if (d.dim == 3) return cells <= 128.0 * d.ne ? kSumBlock / 64 : 1;
+  return largest > 256.0 + d.ne / 4 ? 1 : kSumBlock / kRow;
 }
 
 // Detection blocks of 256 threads (detect_block).

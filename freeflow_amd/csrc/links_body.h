@@ -391,7 +391,11 @@ __device__ __forceinline__ unsigned links_of_element(const unsigned long long* k
   return m;
 }
 
-// Sum of one segment's links by a row of kRow lanes: each lane takes up to two
+// Row sums of a block's kBlock3 / kRow rows.
+using SumPart = double[kBlock3 / kRow][kRow];
+
+// Sum of one segment's links by LANES = kRow lanes, or the block where a
+// window is large (elements_per_block): each lane takes up to two
 // window cells per pass (its own table probes and key rows in flight
 // together), then the links of those cells that name this element, in
 // direction order; a fixed tree folds the lanes.  The pass is a chain of
@@ -399,7 +403,8 @@ __device__ __forceinline__ unsigned links_of_element(const unsigned long long* k
 // with many domains it is bound by instruction issue: one (cell, direction)
 // task per lane loaded every link's force and geometry before knowing whose
 // it was, and folded one element per wave.
-__device__ __forceinline__ void elem_sum2(const LinkArgs& la, const FinalArgs& fa, int elem, int lane) {
+template <int LANES>
+__device__ __forceinline__ void elem_sum2(const LinkArgs& la, const FinalArgs& fa, int elem, int lane, SumPart& part) {
   constexpr int K = 8, STRIDE = elem_stride_v<2>, U = 2;
   const unsigned gen = step_gen(la), tag = step_tag(la);
   const float* v = dev_global(la.v[gen & 1]);
@@ -424,14 +429,14 @@ __device__ __forceinline__ void elem_sum2(const LinkArgs& la, const FinalArgs& f
   const float* lf = dev_global(la.lf);
   const float* lb = dev_global(la.lb);
   const float* lh = dev_global(la.lh);
-  for (int k0 = lane; k0 < ncell; k0 += kRow * U) {
+  for (int k0 = lane; k0 < ncell; k0 += LANES * U) {
     int cell[U];
     unsigned home[U];
     unsigned long long cur[U];
     bool upd[U];
 #pragma unroll
     for (int w = 0; w < U; w++) {
-      const int k = k0 + w * kRow;
+      const int k = k0 + w * LANES;
       upd[w] = false;
       if (k < ncell) {
         const int j = k / wx;
@@ -478,6 +483,18 @@ __device__ __forceinline__ void elem_sum2(const LinkArgs& la, const FinalArgs& f
     }
   }
   row_sums<STRIDE - 1>(acc);
+  if constexpr (LANES > kRow) {  // lane 0 of every row has its sums: fold the rows alike
+    if (lane % kRow == 0) {
+#pragma unroll
+      for (int a = 0; a < STRIDE - 1; a++) part[lane / kRow][a] = acc[a];
+    }
+    __syncthreads();
+    if (lane < kRow) {
+#pragma unroll
+      for (int a = 0; a < STRIDE - 1; a++) acc[a] = part[lane][a];
+    }
+    row_sums<STRIDE - 1>(acc);
+  }
   if (lane == 0) {
     // the element's power: its vertex shares against the velocities the step used
     acc[STRIDE - 1] =
@@ -496,9 +513,8 @@ __device__ __forceinline__ void elem_sum2(const LinkArgs& la, const FinalArgs& f
 // One wave per triangle with (cell, direction) tasks walked the window of a
 // triangle of a sphere of 320 in a serial chain of some 150 loads, which set
 // the launch's time (76 us in a 160x96x96 domain).
-using Sum3Part = double[kBlock3 / kRow][kRow];
 template <int NT>
-__device__ __forceinline__ void elem_sum3(const LinkArgs& la, const FinalArgs& fa, int elem, Sum3Part& part) {
+__device__ __forceinline__ void elem_sum3(const LinkArgs& la, const FinalArgs& fa, int elem, SumPart& part) {
   constexpr int K = 26, STRIDE = elem_stride_v<3>, M = STRIDE - 1, NROW = kBlock3 / kRow;
   static_assert(M <= kRow, "one lane of a row per sum");
   const int tid = (int)threadIdx.x & (NT - 1);
@@ -589,11 +605,7 @@ __device__ __forceinline__ void elem_sum3(const LinkArgs& la, const FinalArgs& f
 template <int DIM>
 union SumsLds {
   DetLds<DIM> det;
-  Sum3Part part[kBlock3 / 64];
-};
-template <>
-union SumsLds<2> {
-  DetLds<2> det;
+  SumPart part[DIM == 2 ? 1 : kBlock3 / 64];
 };
 
 // Second launch of a boundary step, kSumBlock threads per block.  The first
@@ -653,7 +665,8 @@ __device__ __forceinline__ void elem_sums_body(const LinkArgs& la, const FinalAr
   }
   if constexpr (DIM == 2) {
     const int elem = blk * (FB / kRow) + (int)threadIdx.x / kRow;
-    if (elem < la.ne) elem_sum2(la, fa, elem, (int)threadIdx.x % kRow);
+    if (la.epb == 1) elem_sum2<FB>(la, fa, blk, (int)threadIdx.x, lds.part[0]);
+    else if (elem < la.ne) elem_sum2<kRow>(la, fa, elem, (int)threadIdx.x % kRow, lds.part[0]);
   } else if (la.epb == 1) {
     elem_sum3<kBlock3>(la, fa, blk, lds.part[0]);
   } else {

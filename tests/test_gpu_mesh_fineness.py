@@ -1,8 +1,10 @@
-"""3D element sums and link detection by a wave per triangle, which meshes of
-many small triangles take in place of a block per triangle: against the oracle
-(bounds as in test_gpu_boundary_edges), element counts that are no multiple of
-the four waves of a block, windows of one pass of a wave to many and lists that
-overflow; and the same bits as the block form, alone and in a batch."""
+"""Element sums and link detection by the fineness of the mesh, against the
+oracle (bounds as in test_gpu_boundary_edges), alone and in a batch with the
+same bits.  2D: a block per segment where one is long, beside short ones and
+across the grid's edge.  3D: a wave per triangle, which meshes of many small
+triangles take in place of a block per triangle: element counts that are no
+multiple of the four waves of a block, windows of one pass of a wave to many,
+lists that overflow, and the same bits as the block form."""
 import numpy as np
 import pytest
 
@@ -18,6 +20,18 @@ def bodies(*parts):
     off = np.cumsum([0] + [len(p[0]) for p in parts])
     e = np.concatenate([p[1] + o for p, o in zip(parts, off)]).astype(np.uint32)
     return v, e, np.repeat(np.arange(len(parts)), [len(p[1]) for p in parts]).astype(np.int32)
+
+
+@pytest.mark.parametrize("n_seg,r,n_short", [(3, 20.0, 0), (4, 27.3, 0), (5, 44.0, 0), (3, 24.0, 301)])
+def test_long_segments(n_seg, r, n_short):
+    print(f"case long segments {n_seg} r={r} beside {n_short}", flush=True)
+    v, e = wl.cylinder(n_seg, 31.3, 29.6, r)
+    if n_short:
+        v, e, _ = bodies((v, e), wl.cylinder(n_short, 30.2, 28.9, 11.0))
+    vel = np.tile([0.02, -0.01], (len(v), 1))
+    a = run_pair(2, (64, 60, 1), v, vel, e, 3, False)
+    b = run_pair(2, (64, 60, 1), v, vel, e, 3, True)
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
 
 
 @pytest.mark.parametrize("drop,big", [(0, None), (1, None), (2, None), (3, 13.0), (0, 9.0)])
