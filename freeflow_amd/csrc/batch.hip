@@ -368,6 +368,10 @@ static int build_tables(Batch& b, int tile) {
   const int nt = stream_threads(b.dim, tile);
   int rc = grow(&b.d_steps, &b.steps_cap, (size_t)std::max(n, 1));
   if (rc) return rc;
+  std::vector<Grid3> together;  // members with the separable form
+  for (const Domain* d : b.mem)
+    if (sep3d_plan(*d)) together.push_back({d->nx, d->ny, d->nz});
+  const int chunk_planes = batch_chunk_planes(together);
   for (int i = 0; i < n; i++) {
     Domain& d = *b.mem[i];
     DomDev& r = doms[i];
@@ -383,8 +387,9 @@ static int build_tables(Batch& b, int tile) {
     r.bflag = b.d_flag;
     int tx, ty, ntl;
     tiles_of(b, d, tile, &tx, &ty, &ntl);
-    r.chunks = sep3d_plan(d);  // the form the domain has on its own, so its results are the same
-    if (r.chunks) {
+    r.chunks = 0;
+    if (sep3d_plan(d)) {  // the form the domain has on its own, so its results are the same
+      r.chunks = (int)ceil_div(d.nz, chunk_planes);
       tx = (d.nx + kSepTX - 1) / kSepTX;
       ty = (d.ny + kSepTY - 1) / kSepTY;
       ntl = tx * ty * r.chunks;

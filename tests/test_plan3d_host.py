@@ -46,9 +46,9 @@ def plans(tmp_path_factory):
                         "-o", exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     assert r.returncode == 0, r.stdout
 
-    def of(grids):
+    def of(grids, *args):
         text = "".join("%d %d %d\n" % g for g in grids)
-        out = subprocess.run([exe], input=text, stdout=subprocess.PIPE, text=True, check=True).stdout
+        out = subprocess.run([exe, *args], input=text, stdout=subprocess.PIPE, text=True, check=True).stdout
         return [tuple(map(int, line.split())) for line in out.splitlines()]
     return of
 
@@ -62,3 +62,9 @@ def test_chunks_lie_within_the_grid(plans):
     grids = [(nx, ny, nz) for nx in (1, 63, 65, 640) for ny in (1, 7, 130) for nz in (1, 2, 9, 257, 4001)]
     for g, p in zip(grids, plans(grids)):
         assert 0 <= p[0] <= g[2] and 0 <= p[1] <= g[2] and 0 <= p[4] <= g[2], (g, p)
+
+
+def test_chunks_of_a_batch_by_all_its_members(plans):
+    for grids, planes in (([(64, 128, 64)], 4), ([(64, 128, 64)] * 8, 32), ([(64, 128, 64)] * 32, 64), ([], 1),
+                          ([(64, 8, 5), (64, 8, 300)], 2)):
+        assert plans(grids, "batch") == [(planes,)], grids
