@@ -309,7 +309,9 @@ __global__ void __launch_bounds__(kSepThreads, 5)
   const int2 m = map[blockIdx.x];
   if (m.x < 0) return;  // padding of the XCD-aware tile order
   const DomDev* D = doms + m.x;
-  const unsigned p = *D->step & 1u;
+  // uniform to the compiler too: a buffer descriptor that it takes for a lane's
+  // own is applied in a loop over lanes (and 96 VGPRs spill)
+  const unsigned p = (unsigned)__builtin_amdgcn_readfirstlane((int)(*D->step & 1u));
   const LinkArgs& la = D->la;
   sep3d_tile<PERIODIC>(dev_global((const float*)D->mom[p]), dev_global((float*)D->mom[p ^ 1u]), dev_global(la.flags),
                        la.nx, la.ny, la.nz, la.plane, la.omega, D->tiles_x, D->tiles_y, D->chunks, m.y);

@@ -79,8 +79,8 @@ inline int sep3d_chunks(const Grid3& g, size_t plane) {
 // Most planes of a chunk for members that take the separable form together
 // (chunks do not change a bit): each member's own count would cut a batch that
 // fills the chip anyway into chunks of few planes with two more each.  Eight
-// 64x128x64 domains: 146 us a step in chunks of 4, 95 of 32 (the columns 117);
-// 32 of them 562 and 323, 24 of 179x51x42 380 and 231.
+// 64x128x64 domains: 146 us a step in chunks of 4, 85 of 32 (the columns 117);
+// 32 of them 562 and 299, 24 of 179x51x42 380 and 220.
 inline int batch_chunk_planes(const std::vector<Grid3>& members) {
   int best = 1, most = 1;
   for (const Grid3& g : members) most = std::max(most, g.nz);
