@@ -17,9 +17,13 @@
 //
 // The reference clamps every pulled population at zero (FsiCoupling3D.cu:
 // 209-285).  A cell whose populations are positive by the triangle inequality
-// (sep_positive) needs no clamp; a wave with any other cell forms its cells'
+// (sep_bound) needs no clamp; a wave with any other cell forms its cells'
 // populations, and a cell with a negative one goes on with the columns of the
 // clamped ones (sep_clamp), all nine of them.
+// Columns are sums over a cell's populations, so one that is infinite or larger
+// by orders than the others takes them with it, and they would reach all 26
+// neighbours.  Blocks that meet such a cell (not tame) redo the cells around
+// it from single populations (sep_redo).
 #pragma once
 
 #include "ff_internal.h"
@@ -65,19 +69,27 @@ __device__ __forceinline__ SepCoef sep_coef(const float* m) {
   return A;
 }
 
-// Every population of the cell is positive by the triangle inequality: with
-// s = sum |u_a|, p = sum |P_aa|, q = sum |P_ab| (a < b), |H_1| <= 1 and
-// |H_2| <= 2/3, the terms besides rho are at most rho times
+// By the triangle inequality, with s = sum |u_a|, p = sum |P_aa|, q = sum |P_ab|
+// (a < b), |H_1| <= 1 and |H_2| <= 2/3, the terms of a population besides rho
+// are at most rho times
 //   first order 3 s, second order 3 p + 9 q,
 //   third order sum over a != b of 9 |u_b D_a + 2 P_ab u_a| <= 9 s p + 18 s q + 4.5 s^3
-//   (sum u_a^2 |u_b| <= s^3 / 4) and 27 (s q + 2 s^3 / 27),
-// with a margin far above the rounding of this sum.  False for NaN.
-__device__ __forceinline__ bool sep_positive(const float* m) {
+//   (sum u_a^2 |u_b| <= s^3 / 4) and 27 (s q + 2 s^3 / 27).
+// positive: every population of the cell is, with a margin far above the
+// rounding of this sum.  tame: none exceeds rho by more than 256 times (a fluid
+// has s below 1, p and q about s^2).  Both false for NaN and where rho overflows
+// the columns.
+struct SepBound {
+  bool positive, tame;
+};
+__device__ __forceinline__ SepBound sep_bound(const float* m) {
   const float s = fabsf(m[1]) + fabsf(m[2]) + fabsf(m[3]);
   const float p = fabsf(m[4]) + fabsf(m[5]) + fabsf(m[6]);
   const float q = fabsf(m[7]) + fabsf(m[8]) + fabsf(m[9]);
   const float third = fmaf(9.0f, p, fmaf(45.0f, q, 6.5f * s * s));
-  return fmaf(3.0f, s + p, fmaf(9.0f, q, s * third)) < 0.999f && m[0] > 0.0f;
+  const float t = fmaf(3.0f, s + p, fmaf(9.0f, q, s * third));
+  const bool finite = fabsf(m[0]) < 1e30f;
+  return {t < 0.999f && m[0] > 0.0f && finite, t < 256.0f && finite};
 }
 
 // F-, F0, F+ along x of the nine columns of a cell.
@@ -246,6 +258,33 @@ inline int sep3d_plan(const Domain& d) {
   return d.sep_chunks;
 }
 
+// The update of cell (x, y, z) from single populations, in the reference's
+// order, if it pulls from a cell that is not tame; its own thread has stored
+// the columns' result before.
+template <bool PERIODIC>
+__device__ __forceinline__ void sep_redo(const float* __restrict__ in, float* __restrict__ out, int nx, int ny, int nz,
+                                         size_t plane, float omega, int x, int y, int z) {
+  const auto source = [](int g, int n) { return PERIODIC ? (g < 0 ? g + n : (g >= n ? g - n : g)) : min(n - 1, max(0, g)); };
+  float p[27];
+  bool tame = true;
+#pragma unroll
+  for (int i = 0; i < 27; i++) {
+    const int sx = source(x - D3::cx(i), nx), sy = source(y - D3::cy(i), ny), sz = source(z - D3::cz(i), nz);
+    const float* src = in + ((size_t)sz * ny + sy) * nx + sx;
+    float m[10];
+#pragma unroll
+    for (int q = 0; q < 10; q++) m[q] = src[q * plane];
+    tame = tame && sep_bound(m).tame;
+    p[i] = clamp0(recon3_pop(m, i));
+  }
+  if (tame) return;
+  float o[10];
+  collide3(p, omega, o);
+  float* dst = out + ((size_t)z * ny + y) * nx + x;
+#pragma unroll
+  for (int q = 0; q < 10; q++) dst[q * plane] = o[q];
+}
+
 template <bool PERIODIC>
 __device__ __forceinline__ void sep3d_column(const float* __restrict__ in, float* __restrict__ out,
                                              const uint8_t* __restrict__ flags, int nx, int ny, int nz, size_t plane,
@@ -255,6 +294,7 @@ __device__ __forceinline__ void sep3d_column(const float* __restrict__ in, float
   __shared__ float2 s_p[2][3][TY][64], s_m[2][3][TY][64];
   __shared__ float s_p2[2][3][TY][64], s_m2[2][3][TY][64];
   __shared__ __align__(16) float s_side[2][2][TY + 2][kSepSide];  // [buffer][left, right][row + 1][column]
+  __shared__ int s_wild[2];  // a cell that is not tame was met; each cleared by one of the two last waves
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = (int)(threadIdx.x & 63u);
   const int x0 = bx * kSepTX, y0 = by * TY;
@@ -287,13 +327,15 @@ __device__ __forceinline__ void sep3d_column(const float* __restrict__ in, float
       *reinterpret_cast<float4*>(er + k) = *reinterpret_cast<const float4*>(&s_side[buf][1][row + 1][k]);
     }
     // the ninth column (2, 2) is zero unless a clamp acted on a cell or on a side cell
-    const bool plain = sep_positive(m) && el[8] == 0.0f && er[8] == 0.0f;
-    const bool nine = !__all(plain);
+    const SepBound bound = sep_bound(m);
+    const bool plain = bound.positive && el[8] == 0.0f && er[8] == 0.0f;
+    const bool nine = !__all(plain), wild = !__all(bound.tame);
     const SepCoef A = sep_coef(m);
     SepX X;
     sep_columns(A, X);
     refill();  // the moments are used: their registers take the next plane's
     if (nine) {
+      if (wild) s_wild[0] = 1;
       sep_clamp(X.p);
       sep_clamp(X.m);
       sep_clamp(X.c);
@@ -429,6 +471,10 @@ __device__ __forceinline__ void sep3d_column(const float* __restrict__ in, float
       if (i >= 2) out_plane += nxy;
       fout = fz;  // the flag of this step's plane, the next output
     }
+    if ((s_wild[0] || s_wild[1]) && inside) {  // set before the last barrier
+      for (int z = z0; z < zend; z++)
+        if (is_updated(flags[(size_t)z * nxy + cell])) sep_redo<PERIODIC>(in, out, nx, ny, nz, plane, omega, x, y, z);
+    }
   } else {
     const bool upper = wave == TY + 1;  // row TY and the right column, or row -1 and the left column
     const int row = upper ? TY : -1;
@@ -437,12 +483,16 @@ __device__ __forceinline__ void sep3d_column(const float* __restrict__ in, float
     const unsigned soff = (unsigned)(src_y(y0 + srow - 1) * nx + src_x(upper ? x0 + 64 : x0 - 1)) * sizeof(float);
     const float sg = upper ? -1.0f : 1.0f;  // F- of the right column, F+ of the left
     auto side = [&](const float* m, int buf, auto&& refill) {
-      const bool clamp = !__all(sep_positive(m));
+      const SepBound bound = sep_bound(m);
+      const bool clamp = !__all(bound.positive), wild = !__all(bound.tame);
       const SepCoef A = sep_coef(m);
       float f[kSepCols];
       sep_face(A, sg, f);
       refill();
-      if (clamp) sep_clamp(f);
+      if (clamp) {
+        if (wild) s_wild[upper] = 1;
+        sep_clamp(f);
+      }
       if (lane < TY + 2) {
         float* d = s_side[buf][upper ? 1 : 0][lane];
 #pragma unroll
@@ -450,6 +500,7 @@ __device__ __forceinline__ void sep3d_column(const float* __restrict__ in, float
       }
     };
     float m[10], ms[10];
+    s_wild[upper] = 0;
     load(0, soff, ms);
     load(0, off, m);
     side(ms, 0, [&] { load(1, soff, ms); });
