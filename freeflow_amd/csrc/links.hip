@@ -14,9 +14,10 @@
 // Forces: the reference scatters every link force to the element's vertices
 // with float atomicAdd (SolidGeometryProxy_Device.cuh:184-194, 401-421), whose
 // order is nondeterministic.  Here each link force is stored with its link;
-// each element then sums its own links in a fixed order (a row of lanes per
-// segment, a block per triangle), and the finish phase sums elements into vertices (CSR order) and
-// bodies, all in FP64.  Results do not depend on scheduling.
+// each element then sums its own links in a fixed order (a row of lanes or a
+// block per segment, a block or a wave per triangle), and the finish phase sums
+// elements into vertices (CSR order) and bodies, all in FP64.  Results do not
+// depend on scheduling.
 //
 // A step with a boundary is two launches (three when the links must be
 // detected first):
