@@ -52,6 +52,7 @@ struct DomDev {
   int nbc;           // boundary-cell blocks of this domain
   int nvb;           // vertex blocks of the finish phase
   int ndet;          // next-step detection blocks of the element-sum phase
+  int epb, neb;      // elements in a block of that phase, and blocks
   int boundary;
   int chunks;        // z chunks of the separable 3D form, 0: tiles
   int* bflag;        // the batch's overflow flag (set when this domain's table overflowed)
@@ -160,7 +161,7 @@ __global__ void __launch_bounds__(FB) kb_sums(const DomDev* __restrict__ doms, c
   const int2 m = map[blockIdx.x];
   const DomDev* D = doms + m.x;
   __shared__ SumsLds<DIM> lds;
-  elem_sums_body<DIM, S, FB, true>(D->la, D->fa, m.y, D->mom[(*D->step & 1u) ^ 1u], lds);
+  elem_sums_body<DIM, S, FB, true>(D->la, D->fa, m.y, D->mom[(*D->step & 1u) ^ 1u], lds, D->epb, D->neb);
 }
 
 // Per domain: vertex blocks, then one block that folds the wrench, advances
@@ -288,7 +289,7 @@ __global__ void __launch_bounds__(kSumBlock) kb_detect(const DomDev* __restrict_
   const int2 m = map[blockIdx.x];
   const LinkArgs& la = doms[m.x].la;
   __shared__ DetLds<DIM> lds;
-  detect_block<DIM, true>(la, (long long)m.y, step_tag(la), la.v[step_gen(la) & 1u], lds);
+  detect_block<DIM, true>(la, (long long)m.y, step_tag(la), la.v[step_gen(la) & 1u], lds, doms[m.x].epb);
 }
 
 // Block size of the stream launch for a tile index.
@@ -411,10 +412,12 @@ static int build_tables(Batch& b, int tile) {
       r.ndet = detect_blocks(d, true);
       r.fa.copy_blocks = copyback_blocks(d, kSumBlock, 4);  // fewer blocks: many domains share the launch
     } else {
-      r.la.ne = r.la.neb = 0;
+      r.la.ne = 0;
       r.fa.copy_blocks = 0;
     }
-    const int nes = r.la.neb + r.fa.outlet_blocks + r.fa.copy_blocks + r.ndet;
+    r.epb = d.epb;
+    r.neb = bnd ? d.elem_blocks() : 0;
+    const int nes = r.neb + r.fa.outlet_blocks + r.fa.copy_blocks + r.ndet;
     for (int t = 0; t < nes; t++) es.push_back(make_int2(i, t));
     for (int t = 0; t <= r.nvb; t++) fin.push_back(make_int2(i, t));
   }

@@ -392,8 +392,6 @@ LinkArgs link_args(Domain& d, const float* v0, const float* v1, const float* u0,
   la.sb = d.lk_sb;
   la.cap = d.lt_cap;
   la.bc_span = bc_span(d);
-  la.epb = d.epb;
-  la.neb = (d.ne + d.epb - 1) / d.epb;
   la.st = d.st;
   la.gen = d.gen_host;
   la.tag = d.tag_host;

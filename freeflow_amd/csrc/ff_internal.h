@@ -73,7 +73,6 @@ struct LinkArgs {
   float* lh;                  // cap * (Q-1) * DIM  hit point
   float* sb;                  // cap * NM  updated moments of each boundary cell (copied back after the step)
   int cap;
-  int epb, neb;  // elements in a block of the element sums (and of the 3D detection), blocks
   int bc_span;  // link-table slots a boundary-cell block scans per pass (<= its block size)
   StepState* st;
   // Step generation (vertex-buffer parity gen & 1, wrench ring slot) and
@@ -115,7 +114,8 @@ struct Domain {
   int n_outlets = 0;
   // boundary geometry (device, interleaved like the reference proxy)
   int nv = 0, ne = 0, n_bodies = 0;
-  int epb = 1;  // elements in a block of the element sums (LinkArgs)
+  int epb = 1;  // elements in a block of the element sums and of the 3D detection
+  int elem_blocks() const { return (ne + epb - 1) / epb; }
   void* bnd_mem = nullptr;   // one allocation holding the ff_set_boundary arrays below
   void* core_mem = nullptr;  // one allocation holding the moments, flags and reduction scratch
   float* vbuf[2] = {nullptr, nullptr};  // positions by generation parity

@@ -432,7 +432,7 @@ __device__ __forceinline__ bool tri3_t_may_pass(float num, float den) {
 }
 
 // Threads that handle one triangle in the 3D detection and element sums: a
-// block, or a wave (la.epb = 4) where the elements fill the chip anyway.
+// block, or a wave (four elements a block) where the elements fill the chip anyway.
 constexpr int kBlock3 = 256;
 template <int NT>
 __device__ __forceinline__ void group_sync() {
@@ -601,12 +601,12 @@ struct DetLds<3> {
 };
 
 // Detection block of 256 threads: 2D takes blockDim / kRow elements (ROWS) or
-// (element, direction) pairs, 3D la.epb elements.
+// (element, direction) pairs, 3D `epb` elements.
 template <int DIM, bool ROWS>
 __device__ __forceinline__ void detect_block(const LinkArgs& la, long long block, unsigned tag, const float* v,
-                                             DetLds<DIM>& lds) {
+                                             DetLds<DIM>& lds, int epb) {
   if constexpr (DIM == 3) {
-    if (la.epb == 1) {
+    if (epb == 1) {
       if (block < la.ne) build_links_group3<kBlock3>(la, (int)block, tag, v, lds.block);
     } else {
       const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));

@@ -45,10 +45,10 @@ namespace ff {
 
 // ---------------------------------------------------------------- detect
 // Links of the current step under the current tag and vertex buffer.
-template <int DIM>
+template <int DIM, int EPB>
 __global__ void __launch_bounds__(256) k_links_build(LinkArgs la) {
   __shared__ DetLds<DIM> lds;
-  detect_block<DIM, false>(la, blockIdx.x, step_tag(la), la.v[step_gen(la) & 1], lds);
+  detect_block<DIM, false>(la, blockIdx.x, step_tag(la), la.v[step_gen(la) & 1], lds, EPB);
 }
 
 // Links of the current step of a domain stepped on its own (a batch detects
@@ -56,8 +56,9 @@ __global__ void __launch_bounds__(256) k_links_build(LinkArgs la) {
 int launch_detect(Domain& d, const LinkArgs& la) {
   const unsigned g = (unsigned)detect_blocks(d, false);
   if (g > 0) {
-    if (d.dim == 2) k_links_build<2><<<g, 256, 0, d.stream>>>(la);
-    else k_links_build<3><<<g, 256, 0, d.stream>>>(la);
+    if (d.dim == 2) k_links_build<2, 1><<<g, 256, 0, d.stream>>>(la);
+    else if (d.epb == 1) k_links_build<3, 1><<<g, 256, 0, d.stream>>>(la);
+    else k_links_build<3, kSumBlock / 64><<<g, 256, 0, d.stream>>>(la);
   }
   FF_HIP(hipGetLastError());
   return FF_OK;
@@ -65,10 +66,10 @@ int launch_detect(Domain& d, const LinkArgs& la) {
 
 // ---------------------------------------------------------------- sums, finish
 // Element sums, outlets, copy-back and next-step detection.
-template <int DIM, typename S, int FB>
+template <int DIM, typename S, int FB, int EPB>
 __global__ void __launch_bounds__(FB) k_step_sums(LinkArgs la, FinalArgs fa, void* out) {
   __shared__ SumsLds<DIM> lds;
-  elem_sums_body<DIM, S, FB, false>(la, fa, blockIdx.x, out, lds);
+  elem_sums_body<DIM, S, FB, false>(la, fa, blockIdx.x, out, lds, EPB, (la.ne + EPB - 1) / EPB);
 }
 
 // Vertex blocks, then one last block for the body wrenches and the advance
@@ -130,7 +131,7 @@ int elements_per_block(const Domain& d, const float* verts, const uint32_t* elem
 
 // Detection blocks of 256 threads (detect_block).
 int detect_blocks(const Domain& d, bool batched) {
-  if (d.dim == 3) return (d.ne + d.epb - 1) / d.epb;
+  if (d.dim == 3) return d.elem_blocks();
   constexpr int per = 256 / kRow;
   const int n = batched ? d.ne : d.ne * (d.q - 1);  // at most 65536 elements
   return (n + per - 1) / per;
@@ -164,8 +165,13 @@ int launch_step_sums(Domain& d, const LinkArgs& la, void* out, bool detect_next)
   constexpr int FB = kSumBlock;
   const FinalArgs fa = make_final_args(d, out, d.vbuf[0], d.vbuf[1], d.ubuf[0], d.ubuf[1], nullptr);
   const unsigned grid =
-      (unsigned)(la.neb + fa.outlet_blocks + fa.copy_blocks + (detect_next ? detect_blocks(d, false) : 0));
-#define FF_SUM(DIM, S) k_step_sums<DIM, S, FB><<<grid, FB, 0, d.stream>>>(la, fa, out)
+      (unsigned)(d.elem_blocks() + fa.outlet_blocks + fa.copy_blocks + (detect_next ? detect_blocks(d, false) : 0));
+#define FF_SUM(DIM, S)                                                                             \
+  do {                                                                                             \
+    constexpr int many = DIM == 2 ? FB / kRow : FB / 64;                                           \
+    if (d.epb == 1) k_step_sums<DIM, S, FB, 1><<<grid, FB, 0, d.stream>>>(la, fa, out);           \
+    else k_step_sums<DIM, S, FB, many><<<grid, FB, 0, d.stream>>>(la, fa, out);                    \
+  } while (0)
   if (d.dim == 2) {
     if (d.storage == FF_STORAGE_F32) FF_SUM(2, float);
     else if (d.storage == FF_STORAGE_F16) FF_SUM(2, __half);

@@ -346,9 +346,9 @@ __device__ __forceinline__ void wave_block_body(const LinkArgs& la, const FinalA
 // Detection of the next step's links (tag + 1, the next step's vertex
 // positions) into the other link table.
 template <int DIM, bool BATCHED>
-__device__ __forceinline__ void detect_next_body(const LinkArgs& la, int blk, DetLds<DIM>& lds) {
+__device__ __forceinline__ void detect_next_body(const LinkArgs& la, int blk, DetLds<DIM>& lds, int epb) {
   const unsigned gen = step_gen(la);
-  detect_block<DIM, BATCHED>(la, (long long)blk, step_tag(la) + 1u, la.v[(gen + 1u) & 1u], lds);
+  detect_block<DIM, BATCHED>(la, (long long)blk, step_tag(la) + 1u, la.v[(gen + 1u) & 1u], lds, epb);
 }
 
 // ---------------------------------------------------------------- element sums
@@ -609,20 +609,20 @@ union SumsLds {
 };
 
 // Second launch of a boundary step, kSumBlock threads per block.  The first
-// elem_blocks blocks sum links per element (fixed order, FP64) into elem_acc.
+// `neb` blocks sum links per element (fixed order, FP64) into elem_acc.
 // Then outlet blocks: outlet cells of the freshly written buffer
 // (mrApplyOutlet2DKernel / mrApplyOutlet3DKernel; a neighbour that is a
 // boundary cell is read from its side-buffer row, which the copy-back of this
 // launch writes).  Then copy-back blocks: boundary-cell rows into the output.
 // Any further blocks detect the next step's links.
+// `epb` elements a block, a constant in a kernel for one domain, `neb` blocks.
 template <int DIM, typename S, int FB, bool BATCHED>
 __device__ __forceinline__ void elem_sums_body(const LinkArgs& la, const FinalArgs& fa, int blk, void* out,
-                                               SumsLds<DIM>& lds) {
+                                               SumsLds<DIM>& lds, int epb, int neb) {
   static_assert(FB == kSumBlock, "element sums and detection are written for kSumBlock threads");
   constexpr int NM = DIM == 2 ? 6 : 10;
-  const int neb = la.neb;
   if (blk >= neb + fa.outlet_blocks + fa.copy_blocks) {
-    detect_next_body<DIM, BATCHED>(la, blk - neb - fa.outlet_blocks - fa.copy_blocks, lds.det);
+    detect_next_body<DIM, BATCHED>(la, blk - neb - fa.outlet_blocks - fa.copy_blocks, lds.det, epb);
     return;
   }
   if (blk >= neb + fa.outlet_blocks) {
@@ -665,9 +665,9 @@ __device__ __forceinline__ void elem_sums_body(const LinkArgs& la, const FinalAr
   }
   if constexpr (DIM == 2) {
     const int elem = blk * (FB / kRow) + (int)threadIdx.x / kRow;
-    if (la.epb == 1) elem_sum2<FB>(la, fa, blk, (int)threadIdx.x, lds.part[0]);
+    if (epb == 1) elem_sum2<FB>(la, fa, blk, (int)threadIdx.x, lds.part[0]);
     else if (elem < la.ne) elem_sum2<kRow>(la, fa, elem, (int)threadIdx.x % kRow, lds.part[0]);
-  } else if (la.epb == 1) {
+  } else if (epb == 1) {
     elem_sum3<kBlock3>(la, fa, blk, lds.part[0]);
   } else {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
