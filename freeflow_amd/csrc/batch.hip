@@ -73,6 +73,7 @@ struct Batch {
   size_t map_cap = 0;
   unsigned* d_steps = nullptr;
   size_t steps_cap = 0;
+  int epb = -1;  // elements in a block of every member's element sums, 0: they differ, -1: no body
   int n_bc = 0, n_wave = 0, n_bulk = 0, n_sep = 0, n_es = 0, n_fin = 0;
   int* d_flag = nullptr;  // pinned: set by a replay whose detection overflowed a member's link table
   // pending detections (members whose links were not detected ahead): pinned
@@ -156,12 +157,14 @@ __global__ void __launch_bounds__(NT, (KIND == 2 && !DMA ? 4 : 2))
   }
 }
 
-template <int DIM, typename S, int FB>
+// EPB: elements a block of every member, 0 where members differ.
+template <int DIM, typename S, int FB, int EPB>
 __global__ void __launch_bounds__(FB) kb_sums(const DomDev* __restrict__ doms, const int2* __restrict__ map) {
   const int2 m = map[blockIdx.x];
   const DomDev* D = doms + m.x;
   __shared__ SumsLds<DIM> lds;
-  elem_sums_body<DIM, S, FB, true>(D->la, D->fa, m.y, D->mom[(*D->step & 1u) ^ 1u], lds, D->epb, D->neb);
+  elem_sums_body<DIM, S, FB, true>(D->la, D->fa, m.y, D->mom[(*D->step & 1u) ^ 1u], lds, EPB ? EPB : D->epb,
+                                     D->neb);
 }
 
 // Per domain: vertex blocks, then one block that folds the wrench, advances
@@ -239,7 +242,9 @@ void launch_stream_batch(Batch& b, int tile, const int2* map, int nblocks, int n
 template <int DIM, typename S>
 static void launch_tail(Batch& b, const int2* map_sums, const int2* map_fin) {
   constexpr int FB = kSumBlock;
-  if (b.n_es > 0) kb_sums<DIM, S, FB><<<b.n_es, FB, 0, b.stream>>>(b.d_doms, map_sums);
+  constexpr int many = DIM == 2 ? FB / kRow : FB / 64;
+  const auto sums = b.epb == 1 ? kb_sums<DIM, S, FB, 1> : b.epb == 0 ? kb_sums<DIM, S, FB, 0> : kb_sums<DIM, S, FB, many>;
+  if (b.n_es > 0) sums<<<b.n_es, FB, 0, b.stream>>>(b.d_doms, map_sums);
   if (b.n_fin > 0) kb_finish<DIM, 256><<<b.n_fin, 256, 0, b.stream>>>(b.d_doms, map_fin);
 }
 
@@ -375,6 +380,7 @@ static int build_tables(Batch& b, int tile) {
   for (const Domain* d : b.mem)
     if (sep3d_plan(*d)) together.push_back({d->nx, d->ny, d->nz});
   const int chunk_planes = batch_chunk_planes(together);
+  b.epb = -1;
   for (int i = 0; i < n; i++) {
     Domain& d = *b.mem[i];
     DomDev& r = doms[i];
@@ -417,6 +423,7 @@ static int build_tables(Batch& b, int tile) {
     }
     r.epb = d.epb;
     r.neb = bnd ? d.elem_blocks() : 0;
+    if (bnd) b.epb = b.epb < 0 || b.epb == d.epb ? d.epb : 0;
     const int nes = r.neb + r.fa.outlet_blocks + r.fa.copy_blocks + r.ndet;
     for (int t = 0; t < nes; t++) es.push_back(make_int2(i, t));
     for (int t = 0; t <= r.nvb; t++) fin.push_back(make_int2(i, t));

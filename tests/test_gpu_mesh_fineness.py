@@ -67,3 +67,34 @@ def test_wave_and_block_give_the_same_sums():
     assert np.abs(out[0][0]).min() > 0
     for x, y in zip(*out):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+def test_members_of_different_fineness_equal_alone(dim):
+    print(f"case batch of coarse and fine meshes {dim}D", flush=True)
+    grid = (64, 60, 1) if dim == 2 else (36, 33, 32)
+    if dim == 2:
+        meshes = [wl.cylinder(n, 31.3, 29.6, r) for n, r in ((3, 20.0), (60, 12.0), (5, 24.0))]
+    else:
+        meshes = [wl.icosphere([17.3, 16.2, 15.6], r, s) for r, s in ((9.0, 1), (6.5, 3), (4.0, 2))]
+    m = wl.equilibrium_moments(np.random.default_rng(4).uniform(-0.02, 0.02, (int(np.prod(grid)), dim))).astype(np.float32)
+    b = capi.Batch(dim)
+    pairs = []
+    for v, e in meshes:
+        pair = [capi.Domain(dim, *grid, viscosity=0.02) for _ in range(2)]
+        for d in pair:
+            d.set_moments(m)
+            d.set_boundary(v, np.tile([0.02, -0.01, 0.015][:dim], (len(v), 1)), e)
+        b.add(pair[1])
+        pairs.append(pair)
+    b.step(3)
+    b.sync()
+    for alone, member in pairs:
+        alone.step(3)
+        assert np.array_equal(alone.moments(), member.moments())
+        assert np.array_equal(alone.body_wrench(), member.body_wrench()) and np.abs(alone.body_wrench()).min() > 0
+        assert np.array_equal(alone.body_power(), member.body_power())
+    b.close()
+    for pair in pairs:
+        for d in pair:
+            d.close()
